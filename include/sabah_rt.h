@@ -278,19 +278,21 @@ int sabah_moe_prefill_layer(const sabah_moe_layer_desc *layer, const float *d_x,
 int sabah_moe_route(const float *d_logits, int n_tokens, int n_experts, int n_used, int norm_w,
                     float w_scale, int32_t *d_ids, float *d_w, void *stream);
 
-/* How sabah_rt_mul_mat_id_v2 runs IQ3_S, Q4_K and Q6_K calls over many tokens.  No reference
+/* How sabah_rt_mul_mat_id_v2 runs calls over many tokens.  No reference
  * counterpart: the reference's kernel re-reads an expert per (token, slot)
  * (sabah_rt.cu:2791-2839).  Grouped, the (token, slot) pairs are grouped by
  * expert on the device and each expert is read once per call (int8 MFMA);
- * eligible calls have packed rows, dense ids and x, n_experts <= 4096, and
- * k <= 1024 with rows % 64 == 0, or k % 512 == 0, k <= 2048, rows % 32 == 0.
- * mode 0 (default): grouped when eligible with at least 1 (IQ3_S with
- * k <= 1024, and Q6_K) or 2 (otherwise) pairs per expert on average; 1: never;
- * 2: whenever eligible.
- * The results are bit-identical either way.  Grouped calls use library
- * scratch (pair lists, q8 rows) shared by every stream: calls that may
- * overlap on different streams need mode 1 (the token-major kernel uses no
- * scratch).  Returns -1 for another mode. */
+ * eligible calls have packed rows, dense ids and x, n_experts <= 4096 and a
+ * type of Q8_0, Q4_K, Q5_K, Q6_K, IQ3_S, IQ3_XXS, IQ4_NL or IQ4_XS.
+ * mode 0 (default): grouped when eligible with enough pairs per expert on
+ * average (1 or 2, by type and shape); 1: never; 2: whenever eligible.
+ * The results are bit-identical either way.  IQ3_S, Q4_K and Q6_K calls with
+ * k <= 1024, k % 256 == 0 and rows % 64 == 0, or k % 512 == 0, k <= 2048 and rows % 32
+ * == 0, use library scratch (pair lists, q8 rows) shared by every stream when
+ * grouped: such calls that may overlap on different streams need mode 1 (the
+ * token-major kernel uses no scratch).  All other grouped calls use a
+ * workspace of their stream, and inside a stream capture run token-major.
+ * Returns -1 for another mode. */
 int sabah_rt_set_mmid_grouping(int mode);
 
 #ifdef __cplusplus

@@ -1,0 +1,383 @@
+// Group-major expert rows for any row count and any k: the matrix product of
+// an expert's rows with the (token, slot) pairs routed to it, for every 256-element
+// or 32-element format below, with int8 MFMA.  It runs MUL_MAT_ID over
+// many tokens (MMID), a layer's gate/up + SwiGLU (NM = 2) and its down rows.
+//
+// Work split: an item is up to kItemPairs<PT> pairs of one expert
+// (k_group_pairs writes the list); grid = (ceil(rows / 64), items), 256
+// threads.  Wave w owns rows 16 w .. 16 w + 15 of the workgroup's 64 (of each of the
+// NM matrices) over the whole of k, 256 elements per step: the step's weight
+// bytes (coalesced 16-byte chunks) and the pairs' q8 chunks are loaded into
+// registers while the step before is computed, stored to LDS, and each wave
+// decodes its 16 rows' chunk once into MFMA operands for all of the item's
+// 16-pair tiles.  A row's fp32 sum is kept in the lane and grows in block order, so the
+// results are the token-major kernels', bit for bit, in every format.
+#pragma once
+#include "prefill_kernels.h"
+
+namespace sabah {
+
+constexpr int kRowsTile = 64;                 // rows per workgroup and matrix: four waves of 16
+
+// bytes of a row's 256 elements, and the 16-byte chunks that hold them at any
+// alignment, made odd: rows 16 * odd bytes apart start on different LDS banks
+__host__ __device__ constexpr int step_bytes(int qt) { return 256 / block_elems(qt) * block_bytes(qt); }
+__host__ __device__ constexpr int step_chunks(int qt) { return ((15 + step_bytes(qt) + 15) / 16) | 1; }
+// formats paired with 32-element q8_0 blocks: one fp32 term per 32 elements and a
+// last step that may be partial
+__host__ __device__ constexpr bool step_q8_0(int qt) { return act_type(qt) == QT_Q8_0; }
+__host__ __device__ constexpr bool grouped_rows_type(int qt) {
+    return qt == QT_Q8_0 || qt == QT_Q4_K || qt == QT_Q5_K || qt == QT_Q6_K || qt == QT_IQ3_S || qt == QT_IQ3_XXS ||
+           qt == QT_IQ4_NL || qt == QT_IQ4_XS;
+}
+
+// reads at any even LDS address
+struct __attribute__((packed, aligned(2))) LdsU32x {
+    uint32_t v;
+};
+struct __attribute__((packed, aligned(2))) LdsU64x {
+    uint64_t v;
+};
+__device__ inline uint32_t lds_u32x(const uint8_t* p) { return reinterpret_cast<const LdsU32x*>(p)->v; }
+__device__ inline uint64_t lds_u64x(const uint8_t* p) { return reinterpret_cast<const LdsU64x*>(p)->v; }
+__device__ inline uint32_t lds_u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
+// the sums so far are formed here (fewer matrix results live at a time)
+__device__ inline void pin4(int (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(v[i]));
+}
+__device__ inline long op_of(uint32_t lo, uint32_t hi) { return (long)((uint64_t)hi << 32 | lo); }
+
+// 256 elements of the lane's row decoded into MFMA B operands (B[s]: lane
+// quarter q's eight elements 32 s + 8 q .. + 7) with the scales of its
+// sub-blocks.  ns: 32-element blocks of the row left (q8_0 formats): the scale
+// of a block past the row is 0, and so is its term (its activations are zeros).
+template <int QT>
+struct RowOps {
+    long B[8];
+    uint32_t sc[4];               // packed integer scales (Q8_0, IQ4_NL: none)
+    float d[step_q8_0(QT) ? 8 : 2];
+    float mn[2];                  // Q4_K, Q5_K: the mins of items q and q + 4
+};
+
+template <int QT>
+__device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, int ns, RowOps<QT>& O) {
+    if constexpr (QT == QT_IQ3_S) {
+        Iq3sBlockOps I;
+        iq3s_block_ops(unit, tabs, q, I);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) O.B[s] = I.B[s];
+        O.sc[0] = I.ls[0];
+        O.sc[1] = I.ls[1];
+        O.d[0] = h2f(I.d);
+    } else if constexpr (QT == QT_IQ3_XXS) {
+        uint32_t sc[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t aux = lds_u32x(unit + 66 + 4 * s), q2 = lds_u16(unit + 2 + 8 * s + 2 * q);
+            const uint32_t s7 = (aux >> (7 * q)) & 127u;
+            const uint32_t sg = s7 | ((uint32_t)(__builtin_popcount(s7) & 1) << 7);
+            O.B[s] = op_of(lds_u32(tabs, kLdsGrid + 4u * ((q2 & 0xFFu) | ((sg & 15u) << 8))),
+                           lds_u32(tabs, kLdsGrid + 4u * ((q2 >> 8) | ((sg >> 4) << 8))));
+            sc[s] = 2u * (aux >> 28) + 1u;
+        }
+        O.sc[0] = sc[0] | sc[2] << 8 | sc[4] << 16 | sc[6] << 24;
+        O.sc[1] = sc[1] | sc[3] << 8 | sc[5] << 16 | sc[7] << 24;
+        O.d[0] = h2f(lds_u16(unit));
+    } else if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
+        const uint32_t dd = lds_u32x(unit), s0 = lds_u32x(unit + 4), s1 = lds_u32x(unit + 8), s2 = lds_u32x(unit + 12);
+        // get_scale_min_k4 on whole words: items 0..3, then 4..7
+        O.sc[0] = s0 & 0x3F3F3F3Fu;
+        O.sc[1] = (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
+        const uint32_t m0 = s1 & 0x3F3F3F3Fu, m1 = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
+        O.mn[0] = (float)((m0 >> (8 * q)) & 0xFFu);
+        O.mn[1] = (float)((m1 >> (8 * q)) & 0xFFu);
+        O.d[0] = h2f(dd);
+        O.d[1] = h2f(dd >> 16);
+        const uint64_t qh = QT == QT_Q5_K ? lds_u64x(unit + 16 + 8 * q) : 0;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const uint64_t w = lds_u64x(unit + (QT == QT_Q5_K ? 48 : 16) + 32 * p + 8 * q);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                uint64_t v = (w >> (4 * u)) & 0x0F0F0F0F0F0F0F0Full;
+                if constexpr (QT == QT_Q5_K) v |= ((qh >> (2 * p + u)) & 0x0101010101010101ull) << 4;
+                O.B[2 * p + u] = (long)v;
+            }
+        }
+    } else if constexpr (QT == QT_Q6_K) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) O.sc[i] = lds_u32x(unit + 192 + 4 * i);
+        O.d[0] = h2f(lds_u16(unit + 208));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint64_t l0 = lds_u64x(unit + 64 * h + 8 * q), l1 = lds_u64x(unit + 64 * h + 32 + 8 * q);
+            const uint64_t hb = lds_u64x(unit + 128 + 32 * h + 8 * q);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint64_t lo = (t & 1 ? l1 : l0) >> (4 * (t >> 1)), hi = hb >> (2 * t);
+                const uint64_t v = (lo & 0x0F0F0F0F0F0F0F0Full) | ((hi & 0x0303030303030303ull) << 4);
+                // q - 32 per byte, q < 64: q + 96 stays in its byte, and flipping bit 7 takes 128 off
+                const uint32_t a = ((uint32_t)v + 0x60606060u) ^ 0x80808080u;
+                const uint32_t b = ((uint32_t)(v >> 32) + 0x60606060u) ^ 0x80808080u;
+                O.B[4 * h + t] = op_of(a, b);
+            }
+        }
+    } else if constexpr (QT == QT_Q8_0) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            O.B[s] = (long)lds_u64x(unit + 34 * s + 2 + 8 * q);
+            O.d[s] = s < ns ? h2f(lds_u16(unit + 34 * s)) : 0.0f;
+        }
+    } else if constexpr (QT == QT_IQ4_NL) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint64_t n = (lds_u64x(unit + 18 * s + 2 + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
+            O.B[s] = op_of(iq4_levels((uint32_t)n), iq4_levels((uint32_t)(n >> 32)));
+            O.d[s] = s < ns ? h2f(lds_u16(unit + 18 * s)) : 0.0f;
+        }
+    } else {
+        static_assert(QT == QT_IQ4_XS, "a grouped_rows_type");
+        const uint32_t dh = lds_u32x(unit), sl = lds_u32x(unit + 4), sh = dh >> 16;
+        O.d[0] = h2f(dh);
+        O.sc[0] = O.sc[1] = 0;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint64_t n = (lds_u64x(unit + 8 + 16 * s + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
+            O.B[s] = op_of(iq4_levels((uint32_t)n), iq4_levels((uint32_t)(n >> 32)));
+            O.sc[s >> 2] |= (((sl >> (4 * s)) & 15u) | (((sh >> (2 * s)) & 3u) << 4)) << (8 * (s & 3));
+        }
+    }
+}
+
+// acc[i] (the lane's row, pair 4 q + i of a tile) += the step's term(s), the
+// unit dot's integers and fp32 steps in its order.  dx: the tile's activation
+// scales (dx[4 q + i]; q8_0: a row of them per 32 elements, dx_stride apart);
+// bs: Q4_K, Q5_K: this lane's two item sums.
+template <int QT>
+__device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const float* dx, int dx_stride,
+                                 const float (&bs)[2], int q, float (&acc)[4]) {
+    const v4i32 z = {0, 0, 0, 0};
+    if constexpr (step_q8_0(QT)) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const v4i32 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(X[s], O.B[s], z, 0, 0, 0);
+            const float4 dx4 = *reinterpret_cast<const float4*>(dx + s * dx_stride + 4 * q);
+            const float dxv[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn((float)d[i], __fmul_rn(O.d[s], dxv[i])));
+        }
+    } else {
+        const float4 dx4 = *reinterpret_cast<const float4*>(dx + 4 * q);
+        const float dxv[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+        if constexpr (QT == QT_IQ4_XS) {
+            float t[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[i] = __fmul_rn(O.d[0], dxv[i]);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const v4i32 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(X[s], O.B[s], z, 0, 0, 0);
+                const float ls = (float)((int)((O.sc[s >> 2] >> (8 * (s & 3))) & 0xFFu) - 32);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(__fmul_rn(t[i], ls), (float)d[i]));
+            }
+            return;
+        }
+        int isum[4] = {0, 0, 0, 0};
+        if constexpr (QT == QT_Q6_K) {
+            // a scale per 16 elements: two products per sub-block, the other half's weights zero
+            const long first = q < 2 ? -1L : 0L;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const v4i32 da = __builtin_amdgcn_mfma_i32_16x16x32_i8(X[s], O.B[s] & first, z, 0, 0, 0);
+                const v4i32 db = __builtin_amdgcn_mfma_i32_16x16x32_i8(X[s], O.B[s] & ~first, z, 0, 0, 0);
+                const int sa = (int)(int8_t)(O.sc[s >> 1] >> (16 * (s & 1))), sb = (int)(int8_t)(O.sc[s >> 1] >> (16 * (s & 1) + 8));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) isum[i] += __mul24(sa, da[i]) + __mul24(sb, db[i]);   // |da| <= 16 * 32 * 127
+                if (s & 1) pin4(isum);
+            }
+        } else {
+            constexpr bool K = QT == QT_Q4_K || QT == QT_Q5_K;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const v4i32 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(X[s], O.B[s], z, 0, 0, 0);
+                const int ls = (int)(K ? (O.sc[s >> 2] >> (8 * (s & 3))) & 0xFFu : (O.sc[s & 1] >> (8 * (s >> 1))) & 0xFFu);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) isum[i] += __mul24(ls, d[i]);   // |d| <= 32 * 62 * 127
+                if (s == 3) pin4(isum);
+            }
+        }
+        if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
+            // sum mn_j bs_j on fp32 MFMA: exact, every partial sum an integer below 2^24
+            v4f32 ms = {0.0f, 0.0f, 0.0f, 0.0f};
+            ms = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[0], O.mn[0], ms, 0, 0, 0);
+            ms = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[1], O.mn[1], ms, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i] = __fadd_rn(acc[i], __fsub_rn(__fmul_rn(__fmul_rn(O.d[0], dxv[i]), (float)isum[i]),
+                                                     __fmul_rn(__fmul_rn(O.d[1], dxv[i]), ms[i])));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float c = __fmul_rn(__fmul_rn(O.d[0], dxv[i]), (float)isum[i]);
+                if constexpr (QT == QT_IQ3_XXS) c = __fmul_rn(c, 0.25f);
+                acc[i] = __fadd_rn(acc[i], c);
+            }
+        }
+    }
+}
+
+struct GroupedRowsArgs {
+    const uint8_t *w0, *w1;       // bank bases [n_experts][rows][row bytes] (w1: NM = 2's second matrix)
+    size_t expert_stride;
+    const int4* items;            // (expert, first position, pairs, 0); *n_items of them
+    const int* n_items;
+    const int* pair_of;           // pair at each position (MMID, or x_div > 0)
+    int x_div;                    // input row of position p: pair_of[p] / x_div, or p itself (0)
+    const uint8_t* xq;            // q8 rows in MFMA operand order, xq_stride bytes apart
+    int xq_stride;
+    int rows, k;
+    float* out;                   // [position][rows]
+    float* dst;                   // MMID: dst[t][s] rows
+    size_t dst_nb1, dst_nb2;
+    int n_ids;
+};
+
+template <int QT, int NM, int PT, bool MMID>
+__global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a) {
+    constexpr int NT = kThreads, CB = step_bytes(QT), CPR = step_chunks(QT), NC = NM * kRowsTile * CPR;
+    constexpr int NL = (NC + NT - 1) / NT, TP = 16 * PT;
+    constexpr bool Q80 = step_q8_0(QT), BS = QT == QT_Q4_K || QT == QT_Q5_K;
+    typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
+    __shared__ __align__(16) uint8_t tabs[table_bytes(QT) ? table_bytes(QT) : 16];
+    __shared__ __align__(16) uint8_t raw[NL * NT * 16];
+    __shared__ __align__(16) uint8_t xs[TP * kActChunkStride];
+    __shared__ __align__(16) float sdx[(Q80 ? 8 : 1) * TP];
+    __shared__ __align__(16) float sbs[BS ? TP * 8 : 4];
+    __shared__ int spair[TP];
+    const int4 it = a.items[blockIdx.y];
+    if ((int)blockIdx.y >= *a.n_items) return;               // uniform: the list is shorter than its bound
+    const int e = it.x, g0 = it.y, cnt = it.z, nt = (cnt + 15) >> 4;
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int row0 = (int)blockIdx.x * kRowsTile;
+    const int rb = (int)row_bytes(QT, a.k), nch = (a.k + 255) >> 8;
+    const uint8_t* const base0 = a.w0 + (size_t)e * a.expert_stride;
+    const uint8_t* const base1 = NM == 2 ? a.w1 + (size_t)e * a.expert_stride : base0;
+
+    TableRegs<QT, NT> tr = load_tables<QT, NT>(tid);
+    // the thread's 16-byte chunks of a step: chunk j of staged row rw
+    const uint8_t* wp[NL];
+    int wj[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int c = min(tid + NT * i, NC - 1), rw = c / CPR;
+        wj[i] = c - rw * CPR;
+        wp[i] = (NM == 2 && rw >= kRowsTile ? base1 : base0) + (size_t)min(row0 + (rw & (kRowsTile - 1)), a.rows - 1) * rb;
+    }
+    u32x4 wd[NL];
+    auto load_w = [&](int s) {
+        const int len = Q80 ? min(CB, rb - s * CB) : CB;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint8_t* p = wp[i] + (size_t)s * CB;
+            const int lead = (int)(reinterpret_cast<uintptr_t>(p) & 15);
+            wd[i] = *(g_u32x4*)(p - lead + 16 * min(wj[i], (lead + len - 1) >> 4));   // chunks past the row's end repeat its last
+        }
+    };
+    load_w(0);
+    // sixteen threads per pair: 16 bytes of its chunk each, and its scales and sums
+    const ActLayout XL(a.k, Q80 ? QT_Q8_0 : QT_Q8_K);
+    const int xp = tid >> 4, xk = tid & 15;
+    const uint8_t* xrow[PT];
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+        const int pos = g0 + min(16 * p + xp, cnt - 1);
+        xrow[p] = a.xq + (size_t)(a.x_div ? a.pair_of[pos] / a.x_div : pos) * a.xq_stride;
+    }
+    if (MMID && tid < TP) spair[tid] = a.pair_of[g0 + min(tid, cnt - 1)];
+    u32x4 xd[PT];
+    float xdx[PT];
+    uint32_t xbs[PT];
+    // every tile's loads are issued (tiles past the item re-read its last pair): under a
+    // condition the registers they fill end up in scratch memory
+    auto load_xs = [&](int s) {
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+            xd[p] = *reinterpret_cast<const u32x4*>(xrow[p] + s * kActChunkStride + 16 * xk);
+            xdx[p] = reinterpret_cast<const float*>(xrow[p] + XL.off_d)[Q80 ? 8 * s + (xk & 7) : s];
+            if constexpr (BS) xbs[p] = reinterpret_cast<const uint32_t*>(xrow[p] + XL.off_bsum)[8 * s + (xk & 7)];
+        }
+    };
+    load_xs(0);
+    store_tables<QT, NT>(tabs, tr, tid);
+
+    float acc[NM][PT][4];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int p = 0; p < PT; ++p)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[m][p][i] = 0.0f;
+    const size_t my_row = (size_t)min(row0 + 16 * wave + r, a.rows - 1) * rb;
+    for (int s = 0; s < nch; ++s) {
+        if (s) __syncthreads();                              // the step before is computed
+#pragma unroll
+        for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(raw + 16 * (tid + NT * i)) = wd[i];
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+            if (p >= nt) continue;
+            *reinterpret_cast<u32x4*>(xs + (16 * p + xp) * kActChunkStride + 16 * xk) = xd[p];
+            if (Q80 ? xk < 8 : xk == 0) sdx[(Q80 ? TP * xk : 0) + 16 * p + xp] = xdx[p];
+            if (BS && xk < 8)
+                sbs[8 * (16 * p + xp) + xk] = (float)((int)(int16_t)(xbs[p] & 0xFFFFu) + ((int)xbs[p] >> 16));
+        }
+        __syncthreads();
+        if (s + 1 < nch) {
+            load_w(s + 1);
+            load_xs(s + 1);
+        }
+        const int ns = Q80 ? (a.k - 256 * s) >> 5 : 8;
+        RowOps<QT> O[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const uint8_t* g = (m ? base1 : base0) + my_row + (size_t)s * CB;
+            row_ops<QT>(raw + (kRowsTile * m + 16 * wave + r) * (16 * CPR) + (reinterpret_cast<uintptr_t>(g) & 15), tabs, q, ns,
+                        O[m]);
+        }
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+            if (p >= nt) continue;
+            long X[8];
+            const uint8_t* xc = xs + (16 * p + r) * kActChunkStride + 16 * q;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(xc + 64 * t);
+                X[2 * t] = op_of(v.x, v.y);
+                X[2 * t + 1] = op_of(v.z, v.w);
+            }
+            float bs[2] = {0.0f, 0.0f};
+            if constexpr (BS) {
+                bs[0] = sbs[8 * (16 * p + r) + q];
+                bs[1] = sbs[8 * (16 * p + r) + q + 4];
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m) step_term<QT>(O[m], X, sdx + 16 * p, TP, bs, q, acc[m][p]);
+        }
+    }
+    const int row = row0 + 16 * wave + r;
+    if (row >= a.rows) return;
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = 16 * p + 4 * q + i;
+            if (j >= cnt) continue;
+            float v = acc[0][p][i];
+            if constexpr (NM == 2) v = __fmul_rn(silu_f32(v), acc[NM - 1][p][i]);
+            if constexpr (MMID) pair_dst(a.dst, a.dst_nb1, a.dst_nb2, a.n_ids, spair[j])[row] = v;
+            else a.out[(size_t)(g0 + j) * a.rows + row] = v;
+        }
+    }
+}
+
+}  // namespace sabah

@@ -59,6 +59,9 @@ struct GroupArgs {
     float* poison;                // MUL_MAT_ID: a bad pair's dst row becomes NaN (null: none)
     size_t poison_nb1, poison_nb2;  // dst slot and token strides, bytes
     int poison_rows;
+    int4* items;                  // optional: the groups cut into items of at most item_pairs pairs,
+    int* n_items;                 // (expert, first position, pairs, 0), and their number
+    int item_pairs;
 };
 
 // exclusive scan of one int per thread over the workgroup (a multiple of 64
@@ -133,6 +136,15 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
         run += cnt[e];
     }
     if (tid == 0) a.off[E] = total;
+    if (a.items) {                                          // uniform
+        int ni = 0;
+        for (int e = e0; e < e1; ++e) ni += (cnt[e] + a.item_pairs - 1) / a.item_pairs;
+        int at = block_exclusive_scan(ni, tmp, total);
+        for (int e = e0; e < e1; ++e)
+            for (int o = 0; o < cnt[e]; o += a.item_pairs)
+                a.items[at++] = make_int4(e, fill[e] + o, min(a.item_pairs, cnt[e] - o), 0);
+        if (tid == 0) *a.n_items = total;
+    }
     __syncthreads();
     bool bad = false;
     each_pair([&](int p, int e) {
@@ -158,14 +170,14 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
 // floats.  Each workgroup quantises 16 chunk-rows (one per 16-lane row).
 // With `gather`, output row r is input row gather[r] / gdiv, for the rows
 // below *count (the grouped pairs: the rows come out in group order).  With
-// mfma_order (q8_K only), each chunk's bytes are in the grouped kernels'
-// operand order (row16_quant_q8K).
+// mfma_order (q8_K, q8_0), each chunk's bytes are in the grouped kernels'
+// operand order (mfma_chunk_store).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void k_quant_rows(const float* __restrict__ x, int n_rows, int k, int at,
                                                          uint8_t* __restrict__ out, int out_stride,
                                                          const int* __restrict__ gather, int gdiv,
                                                          const int* __restrict__ count, int mfma_order) {
-    const int nch = k / 256;
+    const int nch = (k + 255) / 256;
     const int q = blockIdx.x * (kThreads / 16) + (int)(threadIdx.x >> 4);
     if (q >= n_rows * nch) return;                       // whole 16-lane rows leave together
     const int r = q / nch, c = q - r * nch;

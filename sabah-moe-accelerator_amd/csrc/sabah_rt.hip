@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "dense_kernels.h"
+#include "grouped_rows.h"
 #include "host_decode.h"
 #include "layer_kernels.h"
 #include "mmid_kernels.h"
@@ -97,6 +98,16 @@ Scratch g_scratch_h, g_scratch_hs, g_scratch_ys, g_scratch_hq;
 Scratch g_scratch_sxq, g_scratch_shq, g_scratch_sgl;
 // grouped (prefill) layer: offsets, pair maps, q8 rows of x and h, h and y in group order
 Scratch g_scratch_goff, g_scratch_gpair, g_scratch_gxq, g_scratch_gh, g_scratch_ghq, g_scratch_gy;
+// MUL_MAT_ID through k_grouped_rows: one workspace per stream (calls on
+// different streams may overlap), at most kMaxRowsStreams of them, kept until
+// sabah_rt_shutdown; g_rows_mu is held while a call that uses one is enqueued
+struct RowsWorkspace {
+    hipStream_t st = nullptr;
+    Scratch index, xq;
+};
+constexpr size_t kMaxRowsStreams = 8;
+std::vector<RowsWorkspace> g_rows_ws;
+std::mutex g_rows_mu;
 uint16_t* g_nearest_dev = nullptr;   // IQ3_S encoder table, uploaded on first use
 
 // Optional HIP-event timing of every kernel the library launches, by kernel
@@ -166,6 +177,7 @@ hipStream_t pick_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 // before it fails and names the size (make the same call once outside the
 // capture first).
 std::vector<void*> g_retired;
+std::mutex g_retired_mu;
 size_t g_scratch_total = 0;   // bytes of every grow-only buffer allocated (live and retired)
 
 bool stream_capturing(hipStream_t st) {
@@ -187,6 +199,7 @@ void* grow_scratch(Scratch& s, size_t bytes, hipStream_t stream) {
     size_t want = std::max(bytes, std::max(2 * s.bytes, (size_t)1 << 20));
     void* p = nullptr;
     if (!ck(hipMalloc(&p, want), "scratch allocation")) return nullptr;
+    std::lock_guard<std::mutex> lk(g_retired_mu);
     if (s.p) g_retired.push_back(s.p);
     s.p = p;
     s.bytes = want;
@@ -579,6 +592,13 @@ SABAH_API int sabah_rt_shutdown(void) {
         if (s->p) (void)hipFree(s->p);
         s->p = nullptr;
         s->bytes = 0;
+    }
+    {
+        std::lock_guard<std::mutex> lk(g_rows_mu);
+        for (RowsWorkspace& w : g_rows_ws)
+            for (Scratch* s : {&w.index, &w.xq})
+                if (s->p) (void)hipFree(s->p);
+        g_rows_ws.clear();
     }
     for (void* p : g_retired) (void)hipFree(p);
     g_retired.clear();
@@ -1014,6 +1034,149 @@ static int mmid_grouped(int form, int qt, const uint8_t* bank, size_t expert_str
     return ck(hipGetLastError(), "grouped MUL_MAT_ID launch") ? 0 : -1;
 }
 
+// ---------------------------------------------------------------------------
+// The general grouped form (k_grouped_rows): every format of grouped_rows_type, any
+// k and row count.
+// ---------------------------------------------------------------------------
+// 16-pair tiles per item: four once the experts average 24 pairs, else two
+// (fewer registers, so more waves, where most items are one tile)
+static int rows_tiles(size_t pairs, int n_experts) { return pairs >= 24 * (size_t)n_experts ? 4 : 2; }
+// most items a list of these pairs can hold: one partial item per expert, the rest full
+static size_t rows_item_bound(size_t pairs, int n_experts, int pt) {
+    return std::min(pairs, (size_t)n_experts) + pairs / (size_t)(16 * pt);
+}
+// the grid's second dimension holds the items, and a row offset fits 31 bits
+static bool rows_shape_ok(int qt, size_t pairs, int n_experts, int rows, int k) {
+    return grouped_rows_type(qt) && n_experts <= 4096 && pairs <= (size_t)1 << 24 && row_bytes(qt, k) != 0 &&
+           (size_t)rows * row_bytes(qt, k) < (size_t)1 << 31 && rows_item_bound(pairs, n_experts, 2) <= 65535;
+}
+// a bank every row of which starts at an even address (the decoders' field reads)
+static bool rows_bank_ok(const void* base, size_t expert_stride) {
+    return ((reinterpret_cast<uintptr_t>(base) | expert_stride) & 1) == 0;
+}
+
+// the grouping's buffers in one allocation: items, offsets and the item count, pair maps
+struct RowsIndex {
+    int4* items;
+    int *off, *n_items, *pair_of, *pos_of;
+};
+static size_t rows_index_bytes(size_t pairs, int n_experts, int pt) {
+    return sizeof(int4) * rows_item_bound(pairs, n_experts, pt) + sizeof(int) * ((size_t)n_experts + 2 + 2 * pairs);
+}
+static RowsIndex rows_index(void* p, size_t pairs, int n_experts, int pt) {
+    RowsIndex R;
+    R.items = static_cast<int4*>(p);
+    R.off = reinterpret_cast<int*>(R.items + rows_item_bound(pairs, n_experts, pt));
+    R.n_items = R.off + n_experts + 1;
+    R.pair_of = R.n_items + 1;
+    R.pos_of = R.pair_of + pairs;
+    return R;
+}
+static void launch_group_items(int kind, const RowsIndex& R, const int32_t* d_ids, int n_tokens, int k, int n_experts,
+                               int pt, float* poison, size_t nb1, size_t nb2, int poison_rows, hipStream_t st) {
+    GroupArgs ga{d_ids, n_tokens, k, n_experts, R.off, R.pair_of, R.pos_of, g_err_dev, poison, nb1, nb2, poison_rows,
+                 R.items, R.n_items, 16 * pt};
+    launch_kernel(kind, k_group_pairs, dim3(1), dim3(kGroupThreads), (int)sizeof(int) * (2 * n_experts + kGroupThreads), st,
+                  ga);
+}
+// rows [n][k] -> q8 rows of the weight type's activation format, in MFMA operand order
+static void launch_quant_mfma(int kind, const float* x, size_t n, int k, int qt, uint8_t* out, int stride,
+                              const int* count, hipStream_t st) {
+    const size_t chunks = n * (size_t)((k + 255) / 256);
+    launch_kernel(kind, k_quant_rows, dim3((unsigned)((chunks + 15) / 16)), dim3(kThreads), 0, st, x, (int)n, k,
+                  act_type(qt), out, stride, (const int*)nullptr, 1, count, 1);
+}
+template <int NM, bool MMID>
+static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
+    const dim3 grid((unsigned)((a.rows + kRowsTile - 1) / kRowsTile), (unsigned)items);
+#define SB_ROWS(QT)                                                                                        \
+    case QT:                                                                                               \
+        if (pt == 4) launch_kernel(kind, k_grouped_rows<QT, NM, 4, MMID>, grid, dim3(kThreads), 0, st, a); \
+        else launch_kernel(kind, k_grouped_rows<QT, NM, 2, MMID>, grid, dim3(kThreads), 0, st, a);         \
+        break;
+    switch (qt) {
+    SB_ROWS(QT_Q8_0)
+    SB_ROWS(QT_Q4_K)
+    SB_ROWS(QT_Q5_K)
+    SB_ROWS(QT_Q6_K)
+    SB_ROWS(QT_IQ3_S)
+    SB_ROWS(QT_IQ3_XXS)
+    SB_ROWS(QT_IQ4_NL)
+    SB_ROWS(QT_IQ4_XS)
+    }
+#undef SB_ROWS
+}
+
+// The general grouped form needs at least this many pairs per expert on
+// average, and kRowsMinPairs in all.  Measured (token-major / grouped, us):
+// one layer, top-10 of 512, 2048 / 768: IQ4_XS 178 / 154 at 0.31 pairs per expert,
+// Q5_K 217 / 217 and IQ3_XXS / IQ4_NL 269 / 247 at 0.62, Q8_0 625 / 543 and
+// IQ3_S 336 / 377 at 1.25; top-8 of 128 Q8_0 126 / 144 at 1, 247 / 196 at 2; gate and down
+// nodes cross at the same densities.  Below kRowsMinPairs the grouping's own
+// launches decide: top-2 of 8, 1024 / 2048, a Q8_0 layer 33 / 47 at 16 pairs, 51 / 47 at 32
+// and 158 / 54 at 128, a gate node 17 / 18 at 32 and 55 / 20 at 128.
+constexpr long long kRowsMinPairs = 64;
+static int rows_min_pairs(int qt) { return qt == QT_IQ4_XS || qt == QT_Q5_K || qt == QT_IQ3_XXS ? 1 : 2; }
+static bool rows_worth_it(int qt, long long pairs, int n_experts) {
+    return pairs >= kRowsMinPairs && pairs >= (long long)rows_min_pairs(qt) * n_experts;
+}
+static bool mmid_rows_ok(int qt, bool packed, const uint8_t* bank, size_t expert_stride, size_t ids_id_stride,
+                         size_t ids_token_stride, size_t x_id_stride, size_t x_token_stride, int x_rows, int n_ids,
+                         int n_tokens, int rows, int k, int n_experts) {
+    return packed && ids_id_stride == 4 && ids_token_stride == 4 * (size_t)n_ids && x_id_stride == 4 * (size_t)k &&
+           x_token_stride == 4 * (size_t)k * x_rows && rows_bank_ok(bank, expert_stride) &&
+           rows_shape_ok(qt, (size_t)n_tokens * n_ids, n_experts, rows, k);
+}
+// the stream's workspace, grown to the call's sizes; null: no more streams or
+// no memory (the token-major kernel needs neither)
+static RowsWorkspace* rows_workspace(size_t index_bytes, size_t xq_bytes, hipStream_t st) {
+    RowsWorkspace* w = nullptr;
+    for (RowsWorkspace& v : g_rows_ws)
+        if (v.st == st) w = &v;
+    if (!w) {
+        if (g_rows_ws.size() >= kMaxRowsStreams) return nullptr;
+        g_rows_ws.push_back({});
+        w = &g_rows_ws.back();
+        w->st = st;
+    }
+    return grow_scratch(w->index, index_bytes, st) && grow_scratch(w->xq, xq_bytes, st) ? w : nullptr;
+}
+// 0 done, -1 error, 1 not here: the call takes the token-major kernel.  These
+// calls never take the grouped form inside a capture (a replay would use the stream's
+// workspace outside its order), nor on the per-thread default stream (one
+// handle for every thread's own stream).
+static int mmid_rows(int qt, const uint8_t* bank, size_t expert_stride, const float* d_x, int x_rows,
+                     const int32_t* d_ids, int n_ids, int n_tokens, float* d_dst, size_t dst_id_stride,
+                     size_t dst_token_stride, int rows, int k, int n_experts, hipStream_t st) {
+    if (st == hipStreamPerThread || stream_capturing(st)) return 1;
+    const size_t P = (size_t)n_tokens * n_ids, nx = (size_t)n_tokens * x_rows;
+    const int pt = rows_tiles(P, n_experts), stride = (int)ActLayout(k, act_type(qt)).bytes;
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    RowsWorkspace* w = rows_workspace(rows_index_bytes(P, n_experts, pt), (size_t)stride * nx, st);
+    if (!w) return 1;
+    const RowsIndex R = rows_index(w->index.p, P, n_experts, pt);
+    launch_group_items(KK_MMID, R, d_ids, n_tokens, n_ids, n_experts, pt, d_dst, dst_id_stride, dst_token_stride, rows, st);
+    uint8_t* xq = static_cast<uint8_t*>(w->xq.p);
+    launch_quant_mfma(KK_MMID, d_x, nx, k, qt, xq, stride, nullptr, st);
+    GroupedRowsArgs a{};
+    a.w0 = a.w1 = bank;
+    a.expert_stride = expert_stride;
+    a.items = R.items;
+    a.n_items = R.n_items;
+    a.pair_of = R.pair_of;
+    a.x_div = x_rows == 1 ? n_ids : 1;
+    a.xq = xq;
+    a.xq_stride = stride;
+    a.rows = rows;
+    a.k = k;
+    a.dst = d_dst;
+    a.dst_nb1 = dst_id_stride;
+    a.dst_nb2 = dst_token_stride;
+    a.n_ids = n_ids;
+    launch_rows<1, true>(qt, KK_MMID, pt, rows_item_bound(P, n_experts, pt), a, st);
+    return ck(hipGetLastError(), "grouped MUL_MAT_ID launch") ? 0 : -1;
+}
+
 static uint64_t mix64(uint64_t z) {   // splitmix64's finaliser
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
@@ -1170,48 +1333,55 @@ SABAH_API int sabah_rt_mul_mat_id_v2(const void* source, size_t expert_stride, s
     const int form = mode == 1 ? 0
                    : grouped_mmid_form(qt, packed, ids_id_stride, ids_token_stride, x_id_stride, x_token_stride,
                                        x_rows, n_ids, n_tokens, rows, k, n_experts);
-    if (form && (mode == 2 || (long long)n_tokens * n_ids >= (long long)grouped_min_pairs(form, qt) * n_experts)) {
-        if (mmid_grouped(form, qt, bank, expert_stride, static_cast<const float*>(d_x), x_rows,
-                         static_cast<const int32_t*>(d_ids), n_ids, n_tokens, d_dst, dst_id_stride, dst_token_stride,
-                         rows, k, n_experts, st))
-            return -1;
-        ++g_calls;
-        ++g_grouped_calls;
-        g_tokens += (unsigned long long)n_tokens;
-        g_lookups += (unsigned long long)n_tokens * (unsigned long long)n_ids;
-        selfcheck_call(bank, expert_stride, row_stride, static_cast<const uint8_t*>(d_x), x_id_stride, x_rows,
-                       x_token_stride, static_cast<const uint8_t*>(d_ids), ids_id_stride, ids_token_stride, n_ids,
-                       n_tokens, d_dst, dst_id_stride, dst_token_stride, rows, k, n_experts, qt, st);
-        write_status_file();
-        return 0;
+    const long long pairs = (long long)n_tokens * n_ids;
+    bool grouped = false;
+    if (form) {
+        if (mode == 2 || pairs >= (long long)grouped_min_pairs(form, qt) * n_experts) {
+            if (mmid_grouped(form, qt, bank, expert_stride, static_cast<const float*>(d_x), x_rows,
+                             static_cast<const int32_t*>(d_ids), n_ids, n_tokens, d_dst, dst_id_stride,
+                             dst_token_stride, rows, k, n_experts, st))
+                return -1;
+            grouped = true;
+        }
+    } else if (mode != 1 && (mode == 2 || rows_worth_it(qt, pairs, n_experts)) &&
+               mmid_rows_ok(qt, packed, bank, expert_stride, ids_id_stride, ids_token_stride, x_id_stride,
+                            x_token_stride, x_rows, n_ids, n_tokens, rows, k, n_experts)) {
+        const int rc = mmid_rows(qt, bank, expert_stride, static_cast<const float*>(d_x), x_rows,
+                                 static_cast<const int32_t*>(d_ids), n_ids, n_tokens, d_dst, dst_id_stride,
+                                 dst_token_stride, rows, k, n_experts, st);
+        if (rc < 0) return -1;
+        grouped = rc == 0;
     }
-
-    MmidArgs a{};
-    a.W.base = bank;
-    a.W.ptrs = nullptr;
-    a.W.expert_stride = expert_stride;
-    a.rt.ids = reinterpret_cast<const uint8_t*>(d_ids);
-    a.rt.id_stride = ids_id_stride;
-    a.rt.token_stride = ids_token_stride;
-    a.rt.n_experts = n_experts;
-    a.row_stride = row_stride;
-    a.x = reinterpret_cast<const uint8_t*>(d_x);
-    a.x_id_stride = x_id_stride;
-    a.x_token_stride = x_token_stride;
-    a.x_rows = x_rows;
-    a.n_ids = n_ids;
-    a.n_tokens = n_tokens;
-    a.dst = reinterpret_cast<uint8_t*>(d_dst);
-    a.dst_id_stride = dst_id_stride;
-    a.dst_token_stride = dst_token_stride;
-    a.rows = rows;
-    a.k = k;
-    a.R = rows_mmid(qt, k, packed);
-    if (packed)   // several tokens: longer row tiles in passes (as for the fused layer's kernels)
-        a.R = grow_rows(a.R, rows, (long long)n_ids * n_tokens, kMaxPassesGateUp,
-                        [&](int r) { return launch_lds(qt, make_plan(qt, k, 1, r * contribs_per_row(qt, k))); });
-    a.err = g_err_dev;
-    if (!ck(dispatch_mmid(qt, a, st), "MUL_MAT_ID launch")) return -1;
+    if (grouped) {
+        ++g_grouped_calls;
+    } else {
+        MmidArgs a{};
+        a.W.base = bank;
+        a.W.ptrs = nullptr;
+        a.W.expert_stride = expert_stride;
+        a.rt.ids = reinterpret_cast<const uint8_t*>(d_ids);
+        a.rt.id_stride = ids_id_stride;
+        a.rt.token_stride = ids_token_stride;
+        a.rt.n_experts = n_experts;
+        a.row_stride = row_stride;
+        a.x = reinterpret_cast<const uint8_t*>(d_x);
+        a.x_id_stride = x_id_stride;
+        a.x_token_stride = x_token_stride;
+        a.x_rows = x_rows;
+        a.n_ids = n_ids;
+        a.n_tokens = n_tokens;
+        a.dst = reinterpret_cast<uint8_t*>(d_dst);
+        a.dst_id_stride = dst_id_stride;
+        a.dst_token_stride = dst_token_stride;
+        a.rows = rows;
+        a.k = k;
+        a.R = rows_mmid(qt, k, packed);
+        if (packed)   // several tokens: longer row tiles in passes (as for the fused layer's kernels)
+            a.R = grow_rows(a.R, rows, (long long)n_ids * n_tokens, kMaxPassesGateUp,
+                            [&](int r) { return launch_lds(qt, make_plan(qt, k, 1, r * contribs_per_row(qt, k))); });
+        a.err = g_err_dev;
+        if (!ck(dispatch_mmid(qt, a, st), "MUL_MAT_ID launch")) return -1;
+    }
     ++g_calls;
     g_tokens += (unsigned long long)n_tokens;
     g_lookups += (unsigned long long)n_tokens * (unsigned long long)n_ids;
@@ -1695,9 +1865,46 @@ static int shared_expert_forked(const sabah_moe_layer_desc* L, const float* d_x,
 // shared expert's own launches then run beside the routed gate/up)
 static bool shared_overlaps(const sabah_moe_layer_desc* L, int n_tokens) { return g_side && shared_dense(L, n_tokens); }
 
+// ---------------------------------------------------------------------------
+// A layer over many tokens in the general grouped form (k_grouped_rows), for
+// sabah_moe_layer and the chain.
+// ---------------------------------------------------------------------------
+static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
+    const size_t P = (size_t)n_tokens * n_used;
+    return n_tokens >= 2 && rows_worth_it(L->qt_gate, (long long)P, L->n_experts) &&
+           rows_shape_ok(L->qt_gate, P, L->n_experts, L->d_ff, L->d_model) &&
+           rows_shape_ok(L->qt_down, P, L->n_experts, L->d_model, L->d_ff) &&
+           rows_bank_ok(L->gate, row_bytes(L->qt_gate, L->d_model) * L->d_ff) && rows_bank_ok(L->up, 0) &&
+           rows_bank_ok(L->down, row_bytes(L->qt_down, L->d_ff) * L->d_model);
+}
+static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
+                          int n_used, int n_tokens, float* d_out, const float* d_resid, int pt, hipStream_t st);
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st);
+// 0 done, -1 error, 1 not here (the token-major kernels).  A batch of more
+// than kRowsMaxPairs pairs runs in runs of tokens, so the scratch stays bounded.
+constexpr size_t kRowsMaxPairs = 65536;
+static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
+                          int n_used, int n_tokens, float* d_out, const float* d_resid, hipStream_t st) {
+    if (!rows_layer_ok(L, n_used, n_tokens)) return 1;
+    const int run = std::min(n_tokens, std::max(1, (int)(kRowsMaxPairs / n_used)));
+    const int pt = rows_tiles((size_t)run * n_used, L->n_experts);
+    if (!grouped_layer_ready(L, n_used, run, pt, st)) return 1;
+    for (int t = 0; t < n_tokens; t += run) {
+        const size_t td = (size_t)t * L->d_model, tk = (size_t)t * n_used;
+        const int rc = moe_grouped_on(L, d_x + td, d_ids + tk, d_w + tk, n_used, std::min(run, n_tokens - t), d_out + td,
+                                      d_resid ? d_resid + td : nullptr, pt, st);
+        if (rc) return t ? -1 : rc;
+    }
+    return 0;
+}
+
 static int moe_layer_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                         int n_used, int n_tokens, float* d_out, const float* d_resid, Workspace& ws, hipStream_t st) {
     const int D = L->d_model, F = L->d_ff;
+    if (!ws.arena) {
+        const int rc = moe_layer_rows(L, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, st);
+        if (rc <= 0) return rc;
+    }
     LayerBufs b;
     if (layer_bufs(L, n_used, n_tokens, ws, st, b)) return -1;
     std::unique_lock<std::mutex> side_lock(g_side_mu, std::defer_lock);
@@ -1823,20 +2030,44 @@ static bool grouped_shape_ok(const sabah_moe_layer_desc* L) {
            L->n_experts <= 4096;
 }
 
-static int moe_prefill_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
-                          int n_used, int n_tokens, float* d_out, const float* d_resid, hipStream_t st) {
+// Scratch of a group-major layer.  pt = 0: the fixed-shape kernels' (the
+// pairs' x rows quantised in group order); pt = 2, 4: k_grouped_rows with items of pt
+// 16-pair tiles (one q8 row per token, and the item list).
+struct GroupedBufs {
+    size_t index, xq, h, hq, y;
+};
+static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt) {
+    const size_t P = (size_t)n_tokens * n_used;
+    return {rows_index_bytes(P, L->n_experts, pt ? pt : 2),
+            ActLayout(L->d_model, act_type(L->qt_gate)).bytes * (pt ? (size_t)n_tokens : P), sizeof(float) * P * L->d_ff,
+            ActLayout(L->d_ff, act_type(L->qt_down)).bytes * P, sizeof(float) * P * L->d_model};
+}
+// false inside a capture for which the scratch would have to grow
+static bool grouped_scratch_ready(const GroupedBufs& B, hipStream_t st) {
+    return (g_scratch_goff.bytes >= B.index && g_scratch_gxq.bytes >= B.xq && g_scratch_gh.bytes >= B.h &&
+            g_scratch_ghq.bytes >= B.hq && g_scratch_gy.bytes >= B.y) || !stream_capturing(st);
+}
+
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st) {
+    return grouped_scratch_ready(grouped_bufs(L, n_used, n_tokens, pt), st);
+}
+
+// 0 done, -1 error, 1 (pt > 0 only) nothing launched: no memory for the scratch
+static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
+                          int n_used, int n_tokens, float* d_out, const float* d_resid, int pt, hipStream_t st) {
     const int D = L->d_model, F = L->d_ff, E = L->n_experts;
     const size_t P = (size_t)n_tokens * n_used;
-    const ActLayout XL(D, QT_Q8_K), HL(F, QT_Q8_K);
-    const int xq_stride = (int)XL.bytes, hq_stride = (int)HL.bytes;
-    int* off = static_cast<int*>(grow_scratch(g_scratch_goff, sizeof(int) * (size_t)(E + 1), st));
-    int* pair_of = static_cast<int*>(grow_scratch(g_scratch_gpair, 2 * sizeof(int) * P, st));
-    uint8_t* xq = static_cast<uint8_t*>(grow_scratch(g_scratch_gxq, (size_t)xq_stride * P, st));
-    float* h = static_cast<float*>(grow_scratch(g_scratch_gh, sizeof(float) * P * F, st));
-    uint8_t* hq = static_cast<uint8_t*>(grow_scratch(g_scratch_ghq, (size_t)hq_stride * P, st));
-    float* y = static_cast<float*>(grow_scratch(g_scratch_gy, sizeof(float) * P * D, st));
-    if (!off || !pair_of || !xq || !h || !hq || !y) return -1;
-    int* pos_of = pair_of + P;
+    const int xq_stride = (int)ActLayout(D, act_type(L->qt_gate)).bytes;
+    const int hq_stride = (int)ActLayout(F, act_type(L->qt_down)).bytes;
+    const GroupedBufs B = grouped_bufs(L, n_used, n_tokens, pt);
+    void* index = grow_scratch(g_scratch_goff, B.index, st);
+    uint8_t* xq = static_cast<uint8_t*>(grow_scratch(g_scratch_gxq, B.xq, st));
+    float* h = static_cast<float*>(grow_scratch(g_scratch_gh, B.h, st));
+    uint8_t* hq = static_cast<uint8_t*>(grow_scratch(g_scratch_ghq, B.hq, st));
+    float* y = static_cast<float*>(grow_scratch(g_scratch_gy, B.y, st));
+    if (!index || !xq || !h || !hq || !y) return pt ? 1 : -1;
+    const RowsIndex R = rows_index(index, P, E, pt ? pt : 2);
+    int *const off = R.off, *const pair_of = R.pair_of, *const pos_of = R.pos_of;
     float *hs = nullptr, *shared = nullptr, *sgl = nullptr;
     uint8_t *sxq = nullptr, *shq = nullptr;
     if (L->shared_gate) {
@@ -1862,38 +2093,68 @@ static int moe_prefill_on(const sabah_moe_layer_desc* L, const float* d_x, const
         return -1;
     }
 
-    GroupArgs ga{d_ids, n_tokens, n_used, E, off, pair_of, pos_of, g_err_dev, nullptr, 0, 0, 0};
-    hipLaunchKernelGGL(k_group_pairs, dim3(1), dim3(kGroupThreads), sizeof(int) * (2 * E + kGroupThreads), st, ga);
-    // the pairs' x rows in group order (pair p is token p / n_used)
-    const size_t xq_rows = P * (size_t)(D / 256);
-    hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((xq_rows + 15) / 16)), dim3(kThreads), 0, st, d_x, (int)P, D,
-                       (int)QT_Q8_K, xq, xq_stride, (const int*)pair_of, n_used, (const int*)(off + E), 1);
-    GroupedGateUpArgs gu{};
-    gu.gate = static_cast<const uint8_t*>(L->gate);
-    gu.up = static_cast<const uint8_t*>(L->up);
-    gu.expert_stride = row_bytes(L->qt_gate, D) * (size_t)F;
-    gu.off = off;
-    gu.pair_of = pair_of;
-    gu.k = n_used;
-    gu.xq = xq;
-    gu.xq_stride = xq_stride;
-    gu.h = h;
-    gu.d_model = D;
-    gu.d_ff = F;
-    launch_grouped_gate_up<false>(L->qt_gate, KK_GGATE_UP, dim3((unsigned)(F / kGuRows), (unsigned)E), st, gu);
-    const size_t hq_rows = P * (size_t)(F / 256);
-    hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((hq_rows + 15) / 16)), dim3(kThreads), 0, st, h, (int)P, F,
-                       (int)QT_Q8_K, hq, hq_stride, (const int*)nullptr, 1, (const int*)(off + E), 1);
-    GroupedDownArgs dn{};
-    dn.down = static_cast<const uint8_t*>(L->down);
-    dn.expert_stride = row_bytes(L->qt_down, F) * (size_t)D;
-    dn.off = off;
-    dn.hq = hq;
-    dn.hq_stride = hq_stride;
-    dn.y = y;
-    dn.d_model = D;
-    dn.d_ff = F;
-    launch_grouped_down<false>(L->qt_down, KK_GDOWN, D, E, st, dn);
+    if (pt) {
+        const size_t items = rows_item_bound(P, E, pt);
+        launch_group_items(KK_GGATE_UP, R, d_ids, n_tokens, n_used, E, pt, nullptr, 0, 0, 0, st);
+        launch_quant_mfma(KK_GGATE_UP, d_x, (size_t)n_tokens, D, L->qt_gate, xq, xq_stride, nullptr, st);
+        GroupedRowsArgs ga{};
+        ga.w0 = static_cast<const uint8_t*>(L->gate);
+        ga.w1 = static_cast<const uint8_t*>(L->up);
+        ga.expert_stride = row_bytes(L->qt_gate, D) * (size_t)F;
+        ga.items = R.items;
+        ga.n_items = R.n_items;
+        ga.pair_of = pair_of;
+        ga.x_div = n_used;
+        ga.xq = xq;
+        ga.xq_stride = xq_stride;
+        ga.rows = F;
+        ga.k = D;
+        ga.out = h;
+        launch_rows<2, false>(L->qt_gate, KK_GGATE_UP, pt, items, ga, st);
+        launch_quant_mfma(KK_GDOWN, h, P, F, L->qt_down, hq, hq_stride, off + E, st);
+        ga.w0 = ga.w1 = static_cast<const uint8_t*>(L->down);
+        ga.expert_stride = row_bytes(L->qt_down, F) * (size_t)D;
+        ga.x_div = 0;
+        ga.xq = hq;
+        ga.xq_stride = hq_stride;
+        ga.rows = D;
+        ga.k = F;
+        ga.out = y;
+        launch_rows<1, false>(L->qt_down, KK_GDOWN, pt, items, ga, st);
+    } else {
+        GroupArgs ga{d_ids, n_tokens, n_used, E, off, pair_of, pos_of, g_err_dev, nullptr, 0, 0, 0, nullptr, nullptr, 0};
+        hipLaunchKernelGGL(k_group_pairs, dim3(1), dim3(kGroupThreads), sizeof(int) * (2 * E + kGroupThreads), st, ga);
+        // the pairs' x rows in group order (pair p is token p / n_used)
+        const size_t xq_rows = P * (size_t)(D / 256);
+        hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((xq_rows + 15) / 16)), dim3(kThreads), 0, st, d_x, (int)P, D,
+                           (int)QT_Q8_K, xq, xq_stride, (const int*)pair_of, n_used, (const int*)(off + E), 1);
+        GroupedGateUpArgs gu{};
+        gu.gate = static_cast<const uint8_t*>(L->gate);
+        gu.up = static_cast<const uint8_t*>(L->up);
+        gu.expert_stride = row_bytes(L->qt_gate, D) * (size_t)F;
+        gu.off = off;
+        gu.pair_of = pair_of;
+        gu.k = n_used;
+        gu.xq = xq;
+        gu.xq_stride = xq_stride;
+        gu.h = h;
+        gu.d_model = D;
+        gu.d_ff = F;
+        launch_grouped_gate_up<false>(L->qt_gate, KK_GGATE_UP, dim3((unsigned)(F / kGuRows), (unsigned)E), st, gu);
+        const size_t hq_rows = P * (size_t)(F / 256);
+        hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((hq_rows + 15) / 16)), dim3(kThreads), 0, st, h, (int)P, F,
+                           (int)QT_Q8_K, hq, hq_stride, (const int*)nullptr, 1, (const int*)(off + E), 1);
+        GroupedDownArgs dn{};
+        dn.down = static_cast<const uint8_t*>(L->down);
+        dn.expert_stride = row_bytes(L->qt_down, F) * (size_t)D;
+        dn.off = off;
+        dn.hq = hq;
+        dn.hq_stride = hq_stride;
+        dn.y = y;
+        dn.d_model = D;
+        dn.d_ff = F;
+        launch_grouped_down<false>(L->qt_down, KK_GDOWN, D, E, st, dn);
+    }
     if (join && !ck(hipStreamWaitEvent(st, join, 0), "join the shared expert")) return -1;
     CombineArgs cb{y, pos_of, d_w, shared, d_resid, d_out, n_used, D};
     const bool v4 = D % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_out) | reinterpret_cast<uintptr_t>(d_resid) |
@@ -1924,7 +2185,7 @@ SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const f
     if (n_tokens == 0) return 0;
     ++g_layer_calls;
     g_lookups += (unsigned long long)n_tokens * n_used;
-    return moe_prefill_on(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, pick_stream(stream));
+    return moe_grouped_on(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, 0, pick_stream(stream));
 }
 
 SABAH_API int sabah_moe_route(const float* d_logits, int n_tokens, int n_experts, int n_used, int norm_w,

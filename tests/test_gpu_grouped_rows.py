@@ -1,0 +1,200 @@
+"""The general grouped kernel (k_grouped_rows): MUL_MAT_ID and layers over
+many tokens, for every format it takes, at row counts and k that leave
+partial tiles and a partial last step.
+
+Its integer block sums are exact and its fp32 steps are the token-major
+kernels' in their order, so the bar is bit-identity with the token-major path
+(grouping off, or sabah_moe_layer_noalloc), and the oracle's parity bar.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_bits_equal, assert_parity, random_blocks
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4_K, Q5_K, Q6_K, IQ3_XXS, IQ4_NL, IQ3_S, IQ4_XS = 8, 12, 13, 14, 18, 20, 21, 23
+DEV = torch.device("cuda:0")
+AUTO, NEVER, ALWAYS = 0, 1, 2
+
+
+def T(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def vp(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+@pytest.fixture
+def grouping(hip_rt):
+    lib = hip_rt.lib()
+
+    def set_mode(mode):
+        hip_rt.check(lib.sabah_rt_set_mmid_grouping(mode), "set grouping")
+
+    yield set_mode
+    set_mode(AUTO)
+
+
+def bank_bytes(rng, qt, E, rows, k, scale=0.05):
+    raw = random_blocks(rng, qt, E * rows, k)
+    return raw.reshape(E, rows, -1)
+
+
+def mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped):
+    lib = hip_rt.lib()
+    rb = hip_rt.row_bytes(qt, k)
+    out = torch.full((ids.shape[0], ids.shape[1], rows), 7.0, dtype=torch.float32, device=DEV)
+    before = hip_rt.snapshot()["grouped_calls"]
+    hip_rt.check(lib.sabah_rt_mul_mat_id_v2(
+        vp(bank), ctypes.c_size_t(rows * rb), ctypes.c_size_t(rb),
+        vp(x), ctypes.c_size_t(x.stride(1) * 4), x.shape[1], ctypes.c_size_t(x.stride(0) * 4),
+        vp(ids), ctypes.c_size_t(4), ctypes.c_size_t(ids.stride(0) * 4), ids.shape[1], ids.shape[0],
+        vp(out), ctypes.c_size_t(out.stride(1) * 4), ctypes.c_size_t(out.stride(0) * 4), rows, k, E, qt,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), None), "v2")
+    torch.cuda.synchronize()
+    assert hip_rt.snapshot()["grouped_calls"] == before + int(grouped)
+    return out.cpu().numpy()
+
+
+# (k, rows, tokens): rows below, at and past a 64-row tile, one and several
+# steps of k; 2 tokens leave most experts one pair, 40 give a heavy expert three
+# or more pair tiles (two items), 90 run the four-tile form
+SHAPES = [(256, 17, 2), (768, 64, 40), (1280, 130, 40), (2560, 96, 90)]
+# formats of 32-element blocks: k past a whole 256-step as well
+ODD_K = [(32, 64, 40), (288, 65, 2), (992, 48, 90)]
+
+
+@pytest.mark.parametrize("qt,k,rows,tokens",
+                         [(qt, *s) for qt in (Q8_0, Q4_K, Q5_K, Q6_K, IQ3_XXS, IQ4_NL, IQ3_S, IQ4_XS) for s in SHAPES]
+                         + [(qt, *s) for qt in (Q8_0, IQ4_NL) for s in ODD_K])
+@pytest.mark.parametrize("slot_rows", [False, True])
+def test_grouped_rows_is_bit_identical_to_token_major(hip_rt, orc, grouping, qt, k, rows, tokens, slot_rows):
+    E, K = 7, 3
+    rng = np.random.default_rng(qt * 1000 + k + rows + tokens + slot_rows)
+    raw = bank_bytes(rng, qt, E, rows, k)
+    ids = np.stack([rng.choice(E - 1, K, replace=False) for _ in range(tokens)]).astype(np.int32)
+    ids[:, 0] = 2                                    # a heavy expert; expert E - 1 has no pair
+    ids[1, 2] = ids[1, 0]                            # a duplicate
+    x = rng.standard_normal((tokens, K if slot_rows else 1, k)).astype(np.float32)
+    x[0, 0, :min(k, 256)] = 0.0                      # a block of zeros
+    bank, xd, idd = T(raw), T(x), T(ids)
+    # shapes the fixed-shape grouped kernels take are theirs: off their row multiple here
+    fixed = qt in (Q4_K, Q6_K, IQ3_S) and ((k <= 1024 and rows % 64 == 0) or (k <= 2048 and k % 512 == 0 and rows % 32 == 0))
+    grouping(ALWAYS)
+    got = mmid(hip_rt, bank, qt, rows, k, E, xd, idd, grouped=True)
+    grouping(NEVER)
+    tok = mmid(hip_rt, bank, qt, rows, k, E, xd, idd, grouped=False)
+    assert_bits_equal(got, tok, "qt=%d k=%d rows=%d tokens=%d fixed=%s" % (qt, k, rows, tokens, fixed))
+    if tokens <= 40 and not slot_rows:
+        assert_parity(got, orc.mul_mat_id(raw, x, ids, rows, k, qt), "oracle qt=%d k=%d" % (qt, k))
+
+
+def test_a_bad_id_becomes_nan_and_is_reported(hip_rt, grouping):
+    E, K, rows, k, tokens = 7, 3, 40, 256, 20
+    rng = np.random.default_rng(5)
+    raw = bank_bytes(rng, Q8_0, E, rows, k)
+    ids = rng.integers(0, E, (tokens, K)).astype(np.int32)
+    bad = ids.copy()
+    bad[4, 1] = E
+    x = T(rng.standard_normal((tokens, 1, k)).astype(np.float32))
+    bank = T(raw)
+    grouping(ALWAYS)
+    want = mmid(hip_rt, bank, Q8_0, rows, k, E, x, T(ids), grouped=True)
+    got = mmid(hip_rt, bank, Q8_0, rows, k, E, x, T(bad), grouped=True)
+    assert np.isnan(got[4, 1]).all()
+    got[4, 1] = want[4, 1]
+    assert_bits_equal(got, want, "the other slots")
+    assert hip_rt.lib().sabah_rt_check_errors() == -1
+    assert hip_rt.lib().sabah_rt_check_errors() == 0
+
+
+def test_calls_on_two_streams_and_under_capture(hip_rt, grouping):
+    """Two streams' calls overlap with workspaces of their own, and a captured
+    call (token-major) replays beside them."""
+    E, K, rows, k, tokens = 7, 2, 96, 768, 200
+    rng = np.random.default_rng(6)
+    bank = T(bank_bytes(rng, IQ3_XXS, E, rows, k))
+    xs = [T(rng.standard_normal((tokens, 1, k)).astype(np.float32)) for _ in range(2)]
+    ids = [T(rng.integers(0, E, (tokens, K)).astype(np.int32)) for _ in range(2)]
+    grouping(NEVER)
+    want = [mmid(hip_rt, bank, IQ3_XXS, rows, k, E, xs[i], ids[i], grouped=False) for i in range(2)]
+    grouping(AUTO)
+    lib, rb = hip_rt.lib(), hip_rt.row_bytes(IQ3_XXS, k)
+    outs = [torch.empty(tokens, K, rows, device=DEV) for _ in range(3)]
+
+    def call(i, out, stream):
+        hip_rt.check(lib.sabah_rt_mul_mat_id_v2(
+            vp(bank), ctypes.c_size_t(rows * rb), ctypes.c_size_t(rb), vp(xs[i]), ctypes.c_size_t(k * 4), 1,
+            ctypes.c_size_t(k * 4), vp(ids[i]), ctypes.c_size_t(4), ctypes.c_size_t(K * 4), K, tokens, vp(out),
+            ctypes.c_size_t(rows * 4), ctypes.c_size_t(K * rows * 4), rows, k, E, IQ3_XXS,
+            ctypes.c_void_p(stream.cuda_stream), None), "v2")
+
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    before = hip_rt.snapshot()["grouped_calls"]
+    with torch.cuda.graph(graph):
+        call(0, outs[2], torch.cuda.current_stream())
+    assert hip_rt.snapshot()["grouped_calls"] == before
+    for _ in range(10):
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        for i in range(2):
+            call(i, outs[i], streams[i])
+        torch.cuda.synchronize()
+        for got, i in zip(outs, (0, 1, 0)):
+            assert_bits_equal(got.cpu().numpy(), want[i], "stream %d" % i)
+    assert hip_rt.snapshot()["grouped_calls"] == before + 20
+
+
+def layer(hip_rt, fn, desc, x, ids, w, resid=None):
+    out = torch.full_like(x, float("nan"))
+    hip_rt.check(getattr(hip_rt.lib(), fn)(
+        ctypes.byref(desc), vp(x), vp(ids), vp(w), ids.shape[1], ids.shape[0], vp(out),
+        vp(resid) if resid is not None else None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), fn)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("qtg,qtd,D,F", [(IQ3_XXS, IQ4_NL, 2560, 640), (Q8_0, Q8_0, 288, 96), (Q5_K, IQ4_XS, 512, 256),
+                                         (Q4_K, Q6_K, 256, 1280), (Q6_K, Q8_0, 768, 352), (IQ3_S, IQ3_S, 512, 512)])
+@pytest.mark.parametrize("tokens", [33, 61])
+def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, tokens):
+    from sabah.runtime import rt
+    E, K = 6, 2
+    rng = np.random.default_rng(qtg + qtd + D + tokens)
+    banks = [T(bank_bytes(rng, q, E, rows, k)) for q, rows, k in ((qtg, F, D), (qtg, F, D), (qtd, D, F))]
+    desc = rt.MoeLayerDesc()
+    desc.gate, desc.up, desc.down = (b.data_ptr() for b in banks)
+    desc.qt_gate = desc.qt_up = qtg
+    desc.qt_down = qtd
+    desc.d_model, desc.d_ff, desc.n_experts = D, F, E
+    x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(np.stack([rng.choice(E, K, replace=False) for _ in range(tokens)]).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    for resid in (None, T(rng.standard_normal((tokens, D)).astype(np.float32))):
+        want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x, ids, w, resid)
+        assert_bits_equal(layer(hip_rt, "sabah_moe_layer", desc, x, ids, w, resid), want, "layer")
+    # in place, then captured with the scratch in place
+    y = x.clone()
+    graph = torch.cuda.CUDAGraph()
+    out = torch.empty_like(x)
+    with torch.cuda.graph(graph):
+        hip_rt.check(hip_rt.lib().sabah_moe_layer(
+            ctypes.byref(desc), vp(y), vp(ids), vp(w), K, tokens, vp(out), vp(y),
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "captured layer")
+    want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x, ids, w, x)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
