@@ -3,15 +3,15 @@
 // or 32-element format below, with int8 MFMA.  It runs MUL_MAT_ID over
 // many tokens (MMID), a layer's gate/up + SwiGLU (NM = 2) and its down rows.
 //
-// Work split: an item is up to kItemPairs<PT> pairs of one expert
-// (k_group_pairs writes the list); grid = (ceil(rows / 64), items), 256
-// threads.  Wave w owns rows 16 w .. 16 w + 15 of the workgroup's 64 (of each of the
-// NM matrices) over the whole of k, 256 elements per step: the step's weight
-// bytes (coalesced 16-byte chunks) and the pairs' q8 chunks are loaded into
-// registers while the step before is computed, stored to LDS, and each wave
-// decodes its 16 rows' chunk once into MFMA operands for all of the item's
-// 16-pair tiles.  A row's fp32 sum is kept in the lane and grows in block order, so the
-// results are the token-major kernels', bit for bit, in every format.
+// Work split: an item is up to 16 PT pairs of one expert (k_group_pairs
+// writes the list); grid = (row tiles, items), 256 threads.  A wave owns 16
+// rows, or G = 2 groups of 16 (of one matrix, or the same rows of gate and up), over
+// the whole of k, 256 elements per step: the step's weight bytes (coalesced
+// 16-byte chunks) and the pairs' q8 chunks are loaded into registers while the step
+// before is computed, stored to LDS, and each wave decodes its rows' chunk once into
+// MFMA operands for all of the item's 16-pair tiles.  A row's fp32 sum is kept
+// in the lane and grows in block order, so the results are the token-major
+// kernels', bit for bit, in every format.
 #pragma once
 #include "prefill_kernels.h"
 
@@ -19,10 +19,11 @@ namespace sabah {
 
 constexpr int kRowsTile = 64;                 // rows per workgroup and matrix: four waves of 16
 
-// bytes of a row's 256 elements, and the 16-byte chunks that hold them at any
-// alignment, made odd: rows 16 * odd bytes apart start on different LDS banks
+// bytes of a row's 256 elements, and the 16-byte chunks that hold them at any even
+// address, made odd: rows 16 * odd bytes apart start on different LDS banks
 __host__ __device__ constexpr int step_bytes(int qt) { return 256 / block_elems(qt) * block_bytes(qt); }
-__host__ __device__ constexpr int step_chunks(int qt) { return ((15 + step_bytes(qt) + 15) / 16) | 1; }
+__host__ __device__ constexpr int step_chunks(int qt) { return ((14 + step_bytes(qt) + 15) / 16) | 1; }
+
 // formats paired with 32-element q8_0 blocks: one fp32 term per 32 elements and a
 // last step that may be partial
 __host__ __device__ constexpr bool step_q8_0(int qt) { return act_type(qt) == QT_Q8_0; }
@@ -40,9 +41,23 @@ struct __attribute__((packed, aligned(2))) LdsU64x {
 };
 __device__ inline uint32_t lds_u32x(const uint8_t* p) { return reinterpret_cast<const LdsU32x*>(p)->v; }
 __device__ inline uint64_t lds_u64x(const uint8_t* p) { return reinterpret_cast<const LdsU64x*>(p)->v; }
+// the same through the dwords that hold them and a byte shift, for the formats whose
+// fields start between dwords
+__device__ inline uint32_t lds_u32f(const uint8_t* p) {
+    const uint32_t sh = (uint32_t)reinterpret_cast<uintptr_t>(p) & 3u;
+    const uint32_t* d = reinterpret_cast<const uint32_t*>(p - sh);
+    return __builtin_amdgcn_alignbyte(d[1], d[0], sh);
+}
+__device__ inline uint64_t lds_u64f(const uint8_t* p) {
+    const uint32_t sh = (uint32_t)reinterpret_cast<uintptr_t>(p) & 3u;
+    const uint32_t* d = reinterpret_cast<const uint32_t*>(p - sh);
+    const uint32_t d0 = d[0], d1 = d[1], d2 = d[2];
+    return (uint64_t)__builtin_amdgcn_alignbyte(d2, d1, sh) << 32 | __builtin_amdgcn_alignbyte(d1, d0, sh);
+}
 __device__ inline uint32_t lds_u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
 // the sums so far are formed here (fewer matrix results live at a time)
-__device__ inline void pin4(int (&v)[4]) {
+template <typename V>
+__device__ inline void pin4(V (&v)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(v[i]));
 }
@@ -74,7 +89,7 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
         uint32_t sc[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const uint32_t aux = lds_u32x(unit + 66 + 4 * s), q2 = lds_u16(unit + 2 + 8 * s + 2 * q);
+            const uint32_t aux = lds_u32f(unit + 66 + 4 * s), q2 = lds_u16(unit + 2 + 8 * s + 2 * q);
             const uint32_t s7 = (aux >> (7 * q)) & 127u;
             const uint32_t sg = s7 | ((uint32_t)(__builtin_popcount(s7) & 1) << 7);
             O.B[s] = op_of(lds_u32(tabs, kLdsGrid + 4u * ((q2 & 0xFFu) | ((sg & 15u) << 8))),
@@ -107,12 +122,12 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
         }
     } else if constexpr (QT == QT_Q6_K) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) O.sc[i] = lds_u32x(unit + 192 + 4 * i);
+        for (int i = 0; i < 4; ++i) O.sc[i] = lds_u32f(unit + 192 + 4 * i);
         O.d[0] = h2f(lds_u16(unit + 208));
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const uint64_t l0 = lds_u64x(unit + 64 * h + 8 * q), l1 = lds_u64x(unit + 64 * h + 32 + 8 * q);
-            const uint64_t hb = lds_u64x(unit + 128 + 32 * h + 8 * q);
+            const uint64_t l0 = lds_u64f(unit + 64 * h + 8 * q), l1 = lds_u64f(unit + 64 * h + 32 + 8 * q);
+            const uint64_t hb = lds_u64f(unit + 128 + 32 * h + 8 * q);
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const uint64_t lo = (t & 1 ? l1 : l0) >> (4 * (t >> 1)), hi = hb >> (2 * t);
@@ -126,13 +141,13 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
     } else if constexpr (QT == QT_Q8_0) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            O.B[s] = (long)lds_u64x(unit + 34 * s + 2 + 8 * q);
+            O.B[s] = (long)lds_u64f(unit + 34 * s + 2 + 8 * q);
             O.d[s] = s < ns ? h2f(lds_u16(unit + 34 * s)) : 0.0f;
         }
     } else if constexpr (QT == QT_IQ4_NL) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const uint64_t n = (lds_u64x(unit + 18 * s + 2 + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
+            const uint64_t n = (lds_u64f(unit + 18 * s + 2 + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
             O.B[s] = op_of(iq4_levels((uint32_t)n), iq4_levels((uint32_t)(n >> 32)));
             O.d[s] = s < ns ? h2f(lds_u16(unit + 18 * s)) : 0.0f;
         }
@@ -166,6 +181,7 @@ __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const 
             const float dxv[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn((float)d[i], __fmul_rn(O.d[s], dxv[i])));
+            if (s & 1) pin4(acc);
         }
     } else {
         const float4 dx4 = *reinterpret_cast<const float4*>(dx + 4 * q);
@@ -180,6 +196,7 @@ __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const 
                 const float ls = (float)((int)((O.sc[s >> 2] >> (8 * (s & 3))) & 0xFFu) - 32);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(__fmul_rn(t[i], ls), (float)d[i]));
+                if (s & 1) pin4(acc);
             }
             return;
         }
@@ -228,7 +245,7 @@ __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const 
 }
 
 struct GroupedRowsArgs {
-    const uint8_t *w0, *w1;       // bank bases [n_experts][rows][row bytes] (w1: NM = 2's second matrix)
+    const uint8_t *w0, *w1;       // bank bases [n_experts][rows][row bytes] (w1: up)
     size_t expert_stride;
     const int4* items;            // (expert, first position, pairs, 0); *n_items of them
     const int* n_items;
@@ -243,82 +260,130 @@ struct GroupedRowsArgs {
     int n_ids;
 };
 
-template <int QT, int NM, int PT, bool MMID>
+// what becomes of the sums: out[position][row]; MUL_MAT_ID's dst[t][s][row]; or
+// h = silu(gate) * up, the wave's two row groups being the same rows of two matrices
+enum : int { kRowsOut = 0, kRowsMmid = 1, kRowsSwiglu = 2 };
+
+template <int QT, int G, int PT, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a) {
-    constexpr int NT = kThreads, CB = step_bytes(QT), CPR = step_chunks(QT), NC = NM * kRowsTile * CPR;
-    constexpr int NL = (NC + NT - 1) / NT, TP = 16 * PT;
+    static_assert(MODE != kRowsSwiglu || G == 2, "gate and up");
+    constexpr bool MMID = MODE == kRowsMmid, SWIGLU = MODE == kRowsSwiglu;
+    constexpr int NT = kThreads, CB = step_bytes(QT), CPR = step_chunks(QT);
+    constexpr int NLM = (kRowsTile * CPR + NT - 1) / NT, NL = G * NLM, TP = 16 * PT;   // loads per row group and in all
     constexpr bool Q80 = step_q8_0(QT), BS = QT == QT_Q4_K || QT == QT_Q5_K;
+    // a row's address mod 16 is the same at every step
+    constexpr bool FIXED = CB % 16 == 0;
     typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
     __shared__ __align__(16) uint8_t tabs[table_bytes(QT) ? table_bytes(QT) : 16];
-    __shared__ __align__(16) uint8_t raw[NL * NT * 16];
+    __shared__ __align__(16) uint8_t raw[NL * NT * 16 + 16];   // 16: dwords read past a field's end
     __shared__ __align__(16) uint8_t xs[TP * kActChunkStride];
     __shared__ __align__(16) float sdx[(Q80 ? 8 : 1) * TP];
     __shared__ __align__(16) float sbs[BS ? TP * 8 : 4];
-    __shared__ int spair[TP];
+    __shared__ size_t sdst[MMID ? TP : 1];                   // byte offset of each pair's dst row
     const int4 it = a.items[blockIdx.y];
     if ((int)blockIdx.y >= *a.n_items) return;               // uniform: the list is shorter than its bound
     const int e = it.x, g0 = it.y, cnt = it.z, nt = (cnt + 15) >> 4;
     const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4;
-    const int row0 = (int)blockIdx.x * kRowsTile;
+    const int row0 = (int)blockIdx.x * (SWIGLU ? kRowsTile : G * kRowsTile);
     const int rb = (int)row_bytes(QT, a.k), nch = (a.k + 255) >> 8;
-    const uint8_t* const base0 = a.w0 + (size_t)e * a.expert_stride;
-    const uint8_t* const base1 = NM == 2 ? a.w1 + (size_t)e * a.expert_stride : base0;
+    const uint8_t* base[G];       // of each row group's matrix
+    base[0] = a.w0 + (size_t)e * a.expert_stride;
+    if constexpr (G == 2) base[1] = SWIGLU ? a.w1 + (size_t)e * a.expert_stride : base[0];
+    // row i of the workgroup's group m (rows past the matrix repeat its last)
+    auto row_of = [&](int m, int i) { return min(row0 + (SWIGLU ? 0 : kRowsTile * m) + i, a.rows - 1); };
 
     TableRegs<QT, NT> tr = load_tables<QT, NT>(tid);
-    // the thread's 16-byte chunks of a step: chunk j of staged row rw
-    const uint8_t* wp[NL];
-    int wj[NL];
+    // the thread's i-th 16-byte chunk of a matrix's step: chunk c % CPR of staged row c / CPR,
+    // as an offset from base; len: the step's bytes (chunks past the row's end repeat its last)
+    auto load_off = [&](int m, int i, int s, int len) {
+        const int c = min(tid + NT * i, kRowsTile * CPR - 1), rw = c / CPR;
+        const uint32_t o = (uint32_t)row_of(m, rw) * (uint32_t)rb + (uint32_t)(s * CB);
+        const uint32_t lead = ((uint32_t)reinterpret_cast<uintptr_t>(base[m]) + o) & 15u;
+        return o - lead + 16u * (uint32_t)min(c - rw * CPR, (int)(lead + (uint32_t)len - 1u) >> 4);
+    };
+    uint32_t wf[NL];              // FIXED: load_off at step 0, + 16 (never negative); else the row's offset
+    int wj[FIXED ? 1 : NLM];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-        const int c = min(tid + NT * i, NC - 1), rw = c / CPR;
-        wj[i] = c - rw * CPR;
-        wp[i] = (NM == 2 && rw >= kRowsTile ? base1 : base0) + (size_t)min(row0 + (rw & (kRowsTile - 1)), a.rows - 1) * rb;
+        if constexpr (FIXED) {
+            wf[i] = load_off(i / NLM, i % NLM, 0, CB) + 16u;
+        } else {
+            const int c = min(tid + NT * (i % NLM), kRowsTile * CPR - 1), rw = c / CPR;
+            if (i < NLM) wj[FIXED ? 0 : i] = c - rw * CPR;
+            wf[i] = (uint32_t)row_of(i / NLM, rw) * (uint32_t)rb;
+        }
     }
     u32x4 wd[NL];
     auto load_w = [&](int s) {
-        const int len = Q80 ? min(CB, rb - s * CB) : CB;
+        if constexpr (!FIXED) {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const uint8_t* p = wp[i] + (size_t)s * CB;
-            const int lead = (int)(reinterpret_cast<uintptr_t>(p) & 15);
-            wd[i] = *(g_u32x4*)(p - lead + 16 * min(wj[i], (lead + len - 1) >> 4));   // chunks past the row's end repeat its last
+            for (int i = 0; i < NL; ++i) {
+                const uint32_t o = wf[i] + (uint32_t)(s * CB);
+                const uint32_t lead = ((uint32_t)reinterpret_cast<uintptr_t>(base[i / NLM]) + o) & 15u;
+                const int j = min(wj[FIXED ? 0 : i % NLM], (int)(lead + (uint32_t)CB - 1u) >> 4);
+                wd[i] = *(g_u32x4*)(base[i / NLM] - 16 + (o + 16u - lead + 16u * (uint32_t)j));
+            }
+        } else if (!Q80 || rb - s * CB >= CB) {
+#pragma unroll
+            for (int i = 0; i < NL; ++i) wd[i] = *(g_u32x4*)(base[i / NLM] + (size_t)s * CB - 16 + wf[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+                wd[i] = *(g_u32x4*)(base[i / NLM] - 16 + (load_off(i / NLM, i % NLM, s, rb - s * CB) + 16u));
         }
     };
     load_w(0);
     // sixteen threads per pair: 16 bytes of its chunk each, and its scales and sums
     const ActLayout XL(a.k, Q80 ? QT_Q8_0 : QT_Q8_K);
     const int xp = tid >> 4, xk = tid & 15;
-    const uint8_t* xrow[PT];
+    uint32_t xo[PT];
 #pragma unroll
     for (int p = 0; p < PT; ++p) {
         const int pos = g0 + min(16 * p + xp, cnt - 1);
-        xrow[p] = a.xq + (size_t)(a.x_div ? a.pair_of[pos] / a.x_div : pos) * a.xq_stride;
+        xo[p] = (uint32_t)(a.x_div ? a.pair_of[pos] / a.x_div : pos) * (uint32_t)a.xq_stride;
     }
-    if (MMID && tid < TP) spair[tid] = a.pair_of[g0 + min(tid, cnt - 1)];
+    if (MMID && tid < TP) {
+        const int pr = a.pair_of[g0 + min(tid, cnt - 1)];
+        sdst[tid] = (size_t)(pr / a.n_ids) * a.dst_nb2 + (size_t)(pr % a.n_ids) * a.dst_nb1;
+    }
     u32x4 xd[PT];
     float xdx[PT];
     uint32_t xbs[PT];
     // every tile's loads are issued (tiles past the item re-read its last pair): under a
     // condition the registers they fill end up in scratch memory
     auto load_xs = [&](int s) {
+        const uint8_t *xc = a.xq + s * kActChunkStride, *xd0 = a.xq + XL.off_d + (Q80 ? 32 : 4) * s;
+        const uint8_t* xb = a.xq + XL.off_bsum + 32 * s;
 #pragma unroll
         for (int p = 0; p < PT; ++p) {
-            xd[p] = *reinterpret_cast<const u32x4*>(xrow[p] + s * kActChunkStride + 16 * xk);
-            xdx[p] = reinterpret_cast<const float*>(xrow[p] + XL.off_d)[Q80 ? 8 * s + (xk & 7) : s];
-            if constexpr (BS) xbs[p] = reinterpret_cast<const uint32_t*>(xrow[p] + XL.off_bsum)[8 * s + (xk & 7)];
+            xd[p] = *reinterpret_cast<const u32x4*>(xc + (xo[p] + 16u * (uint32_t)xk));
+            xdx[p] = *reinterpret_cast<const float*>(xd0 + (xo[p] + (Q80 ? 4u * (uint32_t)(xk & 7) : 0u)));
+            if constexpr (BS) xbs[p] = *reinterpret_cast<const uint32_t*>(xb + (xo[p] + 4u * (uint32_t)(xk & 7)));
         }
     };
     load_xs(0);
     store_tables<QT, NT>(tabs, tr, tid);
 
-    float acc[NM][PT][4];
+    float acc[G][PT][4];
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int m = 0; m < G; ++m)
 #pragma unroll
         for (int p = 0; p < PT; ++p)
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[m][p][i] = 0.0f;
-    const size_t my_row = (size_t)min(row0 + 16 * wave + r, a.rows - 1) * rb;
+    uint32_t my_row[G];
+#pragma unroll
+    for (int m = 0; m < G; ++m) my_row[m] = (uint32_t)row_of(m, 16 * wave + r) * (uint32_t)rb;
+    const uint8_t* const xl = xs + r * kActChunkStride + 16 * q;
+    auto read_x = [&](int p, long (&X)[8]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(xl + 16 * p * kActChunkStride + 64 * t);
+            X[2 * t] = op_of(v.x, v.y);
+            X[2 * t + 1] = op_of(v.z, v.w);
+        }
+    };
+#pragma unroll 1
     for (int s = 0; s < nch; ++s) {
         if (s) __syncthreads();                              // the step before is computed
 #pragma unroll
@@ -337,45 +402,43 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a)
             load_xs(s + 1);
         }
         const int ns = Q80 ? (a.k - 256 * s) >> 5 : 8;
-        RowOps<QT> O[NM];
+        long X[8];
+        read_x(0, X);
+        RowOps<QT> O[G];
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const uint8_t* g = (m ? base1 : base0) + my_row + (size_t)s * CB;
-            row_ops<QT>(raw + (kRowsTile * m + 16 * wave + r) * (16 * CPR) + (reinterpret_cast<uintptr_t>(g) & 15), tabs, q, ns,
-                        O[m]);
+        for (int m = 0; m < G; ++m) {
+            const uint32_t lead = ((uint32_t)reinterpret_cast<uintptr_t>(base[m]) + my_row[m] + (uint32_t)(s * CB)) & 15u;
+            row_ops<QT>(raw + NLM * NT * 16 * m + (16 * wave + r) * (16 * CPR) + lead, tabs, q, ns, O[m]);
         }
 #pragma unroll
         for (int p = 0; p < PT; ++p) {
             if (p >= nt) continue;
-            long X[8];
-            const uint8_t* xc = xs + (16 * p + r) * kActChunkStride + 16 * q;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(xc + 64 * t);
-                X[2 * t] = op_of(v.x, v.y);
-                X[2 * t + 1] = op_of(v.z, v.w);
-            }
+            if (p) read_x(p, X);
             float bs[2] = {0.0f, 0.0f};
             if constexpr (BS) {
                 bs[0] = sbs[8 * (16 * p + r) + q];
                 bs[1] = sbs[8 * (16 * p + r) + q + 4];
             }
 #pragma unroll
-            for (int m = 0; m < NM; ++m) step_term<QT>(O[m], X, sdx + 16 * p, TP, bs, q, acc[m][p]);
+            for (int m = 0; m < G; ++m) step_term<QT>(O[m], X, sdx + 16 * p, TP, bs, q, acc[m][p]);
         }
     }
-    const int row = row0 + 16 * wave + r;
-    if (row >= a.rows) return;
 #pragma unroll
-    for (int p = 0; p < PT; ++p) {
+    for (int m = 0; m < (SWIGLU ? 1 : G); ++m) {
+        const int row = row0 + kRowsTile * m + 16 * wave + r;
+        if (row >= a.rows) break;
+        float* const out = MMID ? nullptr : a.out + (size_t)(g0 + 4 * q) * a.rows + row;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int j = 16 * p + 4 * q + i;
-            if (j >= cnt) continue;
-            float v = acc[0][p][i];
-            if constexpr (NM == 2) v = __fmul_rn(silu_f32(v), acc[NM - 1][p][i]);
-            if constexpr (MMID) pair_dst(a.dst, a.dst_nb1, a.dst_nb2, a.n_ids, spair[j])[row] = v;
-            else a.out[(size_t)(g0 + j) * a.rows + row] = v;
+        for (int p = 0; p < PT; ++p) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = 16 * p + 4 * q + i;
+                if (j >= cnt) continue;
+                float v = acc[m][p][i];
+                if constexpr (SWIGLU) v = __fmul_rn(silu_f32(v), acc[G - 1][p][i]);
+                if constexpr (MMID) *reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.dst) + sdst[j] + 4 * (size_t)row) = v;
+                else out[(size_t)(16 * p + i) * a.rows] = v;
+            }
         }
     }
 }

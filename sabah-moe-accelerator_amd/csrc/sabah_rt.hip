@@ -1038,9 +1038,15 @@ static int mmid_grouped(int form, int qt, const uint8_t* bank, size_t expert_str
 // The general grouped form (k_grouped_rows): every format of grouped_rows_type, any
 // k and row count.
 // ---------------------------------------------------------------------------
-// 16-pair tiles per item: four once the experts average 24 pairs, else two
-// (fewer registers, so more waves, where most items are one tile)
-static int rows_tiles(size_t pairs, int n_experts) { return pairs >= 24 * (size_t)n_experts ? 4 : 2; }
+// 16-pair tiles per item: four where the experts average 24 pairs and the
+// launch still fills the chip, else two (fewer registers, so more waves, where most
+// items are one tile).  Measured (two / four tiles, us): a Q4_K / Q6_K layer at 125 pairs
+// per expert 586 / 512, Q5_K at 32 210 / 198, Q8_0 at 16 199 / 238, IQ3_XXS /
+// IQ4_NL at 10 543 / 635; a Q8_0 down node over 8 experts (1,024 rows, 75 pairs each) 33 / 36.
+static int rows_tiles(size_t pairs, int n_experts, int rows) {
+    const size_t items = pairs / 64 + std::min(pairs, (size_t)n_experts);
+    return pairs >= 24 * (size_t)n_experts && (size_t)(rows / kRowsTile) * items >= 1024 ? 4 : 2;
+}
 // most items a list of these pairs can hold: one partial item per expert, the rest full
 static size_t rows_item_bound(size_t pairs, int n_experts, int pt) {
     return std::min(pairs, (size_t)n_experts) + pairs / (size_t)(16 * pt);
@@ -1048,7 +1054,8 @@ static size_t rows_item_bound(size_t pairs, int n_experts, int pt) {
 // the grid's second dimension holds the items, and a row offset fits 31 bits
 static bool rows_shape_ok(int qt, size_t pairs, int n_experts, int rows, int k) {
     return grouped_rows_type(qt) && n_experts <= 4096 && pairs <= (size_t)1 << 24 && row_bytes(qt, k) != 0 &&
-           (size_t)rows * row_bytes(qt, k) < (size_t)1 << 31 && rows_item_bound(pairs, n_experts, 2) <= 65535;
+           (size_t)rows * row_bytes(qt, k) < (size_t)1 << 31 &&
+           pairs * ActLayout(k, act_type(qt)).bytes < (size_t)1 << 32 && rows_item_bound(pairs, n_experts, 2) <= 65535;
 }
 // a bank every row of which starts at an even address (the decoders' field reads)
 static bool rows_bank_ok(const void* base, size_t expert_stride) {
@@ -1086,13 +1093,22 @@ static void launch_quant_mfma(int kind, const float* x, size_t n, int k, int qt,
     launch_kernel(kind, k_quant_rows, dim3((unsigned)((chunks + 15) / 16)), dim3(kThreads), 0, st, x, (int)n, k,
                   act_type(qt), out, stride, (const int*)nullptr, 1, count, 1);
 }
-template <int NM, bool MMID>
-static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
-    const dim3 grid((unsigned)((a.rows + kRowsTile - 1) / kRowsTile), (unsigned)items);
-#define SB_ROWS(QT)                                                                                        \
-    case QT:                                                                                               \
-        if (pt == 4) launch_kernel(kind, k_grouped_rows<QT, NM, 4, MMID>, grid, dim3(kThreads), 0, st, a); \
-        else launch_kernel(kind, k_grouped_rows<QT, NM, 2, MMID>, grid, dim3(kThreads), 0, st, a);         \
+// Two 16-row groups per wave (128-row tiles, the activations read from LDS
+// once for both) for two-tile items, where 128-row tiles fit the rows and the launch
+// still fills the chip.  Measured (one / two groups, us): an IQ3_XXS / IQ4_NL layer 582 /
+// 543, IQ4_XS 472 / 429, IQ3_S 583 / 535; Q8_0 199 / 203, and with four tiles Q4_K / Q6_K 512 / 525.
+static int rows_groups(int qt, int pt, int rows, size_t items) {
+    const int tiles = (rows + 2 * kRowsTile - 1) / (2 * kRowsTile);
+    return qt != QT_Q8_0 && pt == 2 && tiles * 2 * kRowsTile <= rows + rows / 8 && (size_t)tiles * items >= 1024 ? 2 : 1;
+}
+template <int G, int MODE>
+static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
+    const int tile = MODE == kRowsSwiglu ? kRowsTile : G * kRowsTile;
+    const dim3 grid((unsigned)((a.rows + tile - 1) / tile), (unsigned)items);
+#define SB_ROWS(QT)                                                                                       \
+    case QT:                                                                                              \
+        if (pt == 4) launch_kernel(kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a); \
+        else launch_kernel(kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);         \
         break;
     switch (qt) {
     SB_ROWS(QT_Q8_0)
@@ -1105,6 +1121,12 @@ static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRow
     SB_ROWS(QT_IQ4_XS)
     }
 #undef SB_ROWS
+}
+template <int MODE>
+static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
+    if constexpr (MODE == kRowsSwiglu) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st);
+    else if (rows_groups(qt, pt, a.rows, items) == 2) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st);
+    else launch_rows_g<1, MODE>(qt, kind, pt, items, a, st);
 }
 
 // The general grouped form needs at least this many pairs per expert on
@@ -1150,7 +1172,7 @@ static int mmid_rows(int qt, const uint8_t* bank, size_t expert_stride, const fl
                      size_t dst_token_stride, int rows, int k, int n_experts, hipStream_t st) {
     if (st == hipStreamPerThread || stream_capturing(st)) return 1;
     const size_t P = (size_t)n_tokens * n_ids, nx = (size_t)n_tokens * x_rows;
-    const int pt = rows_tiles(P, n_experts), stride = (int)ActLayout(k, act_type(qt)).bytes;
+    const int pt = rows_tiles(P, n_experts, rows), stride = (int)ActLayout(k, act_type(qt)).bytes;
     std::lock_guard<std::mutex> lk(g_rows_mu);
     RowsWorkspace* w = rows_workspace(rows_index_bytes(P, n_experts, pt), (size_t)stride * nx, st);
     if (!w) return 1;
@@ -1173,7 +1195,7 @@ static int mmid_rows(int qt, const uint8_t* bank, size_t expert_stride, const fl
     a.dst_nb1 = dst_id_stride;
     a.dst_nb2 = dst_token_stride;
     a.n_ids = n_ids;
-    launch_rows<1, true>(qt, KK_MMID, pt, rows_item_bound(P, n_experts, pt), a, st);
+    launch_rows<kRowsMmid>(qt, KK_MMID, pt, rows_item_bound(P, n_experts, pt), a, st);
     return ck(hipGetLastError(), "grouped MUL_MAT_ID launch") ? 0 : -1;
 }
 
@@ -1869,8 +1891,12 @@ static bool shared_overlaps(const sabah_moe_layer_desc* L, int n_tokens) { retur
 // A layer over many tokens in the general grouped form (k_grouped_rows), for
 // sabah_moe_layer and the chain.
 // ---------------------------------------------------------------------------
+// A batch of more than kRowsMaxPairs pairs runs in runs of tokens, so the
+// scratch stays bounded.
+constexpr size_t kRowsMaxPairs = 65536;
+static int rows_run(int n_used, int n_tokens) { return std::min(n_tokens, std::max(1, (int)(kRowsMaxPairs / n_used))); }
 static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
-    const size_t P = (size_t)n_tokens * n_used;
+    const size_t P = (size_t)rows_run(n_used, n_tokens) * n_used;
     return n_tokens >= 2 && rows_worth_it(L->qt_gate, (long long)P, L->n_experts) &&
            rows_shape_ok(L->qt_gate, P, L->n_experts, L->d_ff, L->d_model) &&
            rows_shape_ok(L->qt_down, P, L->n_experts, L->d_model, L->d_ff) &&
@@ -1880,14 +1906,12 @@ static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_token
 static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                           int n_used, int n_tokens, float* d_out, const float* d_resid, int pt, hipStream_t st);
 static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st);
-// 0 done, -1 error, 1 not here (the token-major kernels).  A batch of more
-// than kRowsMaxPairs pairs runs in runs of tokens, so the scratch stays bounded.
-constexpr size_t kRowsMaxPairs = 65536;
+// 0 done, -1 error, 1 not here (the token-major kernels)
 static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                           int n_used, int n_tokens, float* d_out, const float* d_resid, hipStream_t st) {
     if (!rows_layer_ok(L, n_used, n_tokens)) return 1;
-    const int run = std::min(n_tokens, std::max(1, (int)(kRowsMaxPairs / n_used)));
-    const int pt = rows_tiles((size_t)run * n_used, L->n_experts);
+    const int run = rows_run(n_used, n_tokens);
+    const int pt = rows_tiles((size_t)run * n_used, L->n_experts, L->d_ff);
     if (!grouped_layer_ready(L, n_used, run, pt, st)) return 1;
     for (int t = 0; t < n_tokens; t += run) {
         const size_t td = (size_t)t * L->d_model, tk = (size_t)t * n_used;
@@ -2110,7 +2134,7 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
         ga.rows = F;
         ga.k = D;
         ga.out = h;
-        launch_rows<2, false>(L->qt_gate, KK_GGATE_UP, pt, items, ga, st);
+        launch_rows<kRowsSwiglu>(L->qt_gate, KK_GGATE_UP, pt, items, ga, st);
         launch_quant_mfma(KK_GDOWN, h, P, F, L->qt_down, hq, hq_stride, off + E, st);
         ga.w0 = ga.w1 = static_cast<const uint8_t*>(L->down);
         ga.expert_stride = row_bytes(L->qt_down, F) * (size_t)D;
@@ -2120,7 +2144,7 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
         ga.rows = D;
         ga.k = F;
         ga.out = y;
-        launch_rows<1, false>(L->qt_down, KK_GDOWN, pt, items, ga, st);
+        launch_rows<kRowsOut>(L->qt_down, KK_GDOWN, pt, items, ga, st);
     } else {
         GroupArgs ga{d_ids, n_tokens, n_used, E, off, pair_of, pos_of, g_err_dev, nullptr, 0, 0, 0, nullptr, nullptr, 0};
         hipLaunchKernelGGL(k_group_pairs, dim3(1), dim3(kGroupThreads), sizeof(int) * (2 * E + kGroupThreads), st, ga);

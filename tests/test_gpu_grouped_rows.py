@@ -65,8 +65,9 @@ def mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped):
 
 # (k, rows, tokens): rows below, at and past a 64-row tile, one and several
 # steps of k; 2 tokens leave most experts one pair, 40 give a heavy expert three
-# or more pair tiles (two items), 90 run the four-tile form
-SHAPES = [(256, 17, 2), (768, 64, 40), (1280, 130, 40), (2560, 96, 90)]
+# or more pair tiles (two items); 6200 rows make 90 tokens' items four-tile ones, 13240
+# rows give each wave two row groups
+SHAPES = [(256, 17, 2), (768, 64, 40), (1280, 130, 40), (2560, 96, 90), (512, 6200, 90), (256, 13240, 40)]
 # formats of 32-element blocks: k past a whole 256-step as well
 ODD_K = [(32, 64, 40), (288, 65, 2), (992, 48, 90)]
 
@@ -85,14 +86,12 @@ def test_grouped_rows_is_bit_identical_to_token_major(hip_rt, orc, grouping, qt,
     x = rng.standard_normal((tokens, K if slot_rows else 1, k)).astype(np.float32)
     x[0, 0, :min(k, 256)] = 0.0                      # a block of zeros
     bank, xd, idd = T(raw), T(x), T(ids)
-    # shapes the fixed-shape grouped kernels take are theirs: off their row multiple here
-    fixed = qt in (Q4_K, Q6_K, IQ3_S) and ((k <= 1024 and rows % 64 == 0) or (k <= 2048 and k % 512 == 0 and rows % 32 == 0))
     grouping(ALWAYS)
     got = mmid(hip_rt, bank, qt, rows, k, E, xd, idd, grouped=True)
     grouping(NEVER)
     tok = mmid(hip_rt, bank, qt, rows, k, E, xd, idd, grouped=False)
-    assert_bits_equal(got, tok, "qt=%d k=%d rows=%d tokens=%d fixed=%s" % (qt, k, rows, tokens, fixed))
-    if tokens <= 40 and not slot_rows:
+    assert_bits_equal(got, tok, "qt=%d k=%d rows=%d tokens=%d" % (qt, k, rows, tokens))
+    if rows <= 130 and tokens <= 40 and not slot_rows:
         assert_parity(got, orc.mul_mat_id(raw, x, ids, rows, k, qt), "oracle qt=%d k=%d" % (qt, k))
 
 
@@ -166,7 +165,8 @@ def layer(hip_rt, fn, desc, x, ids, w, resid=None):
 
 
 @pytest.mark.parametrize("qtg,qtd,D,F", [(IQ3_XXS, IQ4_NL, 2560, 640), (Q8_0, Q8_0, 288, 96), (Q5_K, IQ4_XS, 512, 256),
-                                         (Q4_K, Q6_K, 256, 1280), (Q6_K, Q8_0, 768, 352), (IQ3_S, IQ3_S, 512, 512)])
+                                         (Q4_K, Q6_K, 256, 1280), (Q6_K, Q8_0, 768, 352), (IQ3_S, IQ3_S, 512, 512),
+                                         (IQ3_XXS, IQ4_NL, 16640, 64)])
 @pytest.mark.parametrize("tokens", [33, 61])
 def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, tokens):
     from sabah.runtime import rt
