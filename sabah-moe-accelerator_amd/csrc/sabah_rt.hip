@@ -1043,7 +1043,9 @@ static int mmid_grouped(int form, int qt, const uint8_t* bank, size_t expert_str
 // items are one tile).  Measured (two / four tiles, us): a Q4_K / Q6_K layer at 125 pairs
 // per expert 586 / 512, Q5_K at 32 210 / 198, Q8_0 at 16 199 / 238, IQ3_XXS /
 // IQ4_NL at 10 543 / 635; a Q8_0 down node over 8 experts (1,024 rows, 75 pairs each) 33 / 36.
-static int rows_tiles(size_t pairs, int n_experts, int rows) {
+// Q8_0 gate/up has no four-tile form: it would spill registers.
+static int rows_tiles(size_t pairs, int n_experts, int rows, bool q8_0_pair = false) {
+    if (q8_0_pair) return 2;
     const size_t items = pairs / 64 + std::min(pairs, (size_t)n_experts);
     return pairs >= 24 * (size_t)n_experts && (size_t)(rows / kRowsTile) * items >= 1024 ? 4 : 2;
 }
@@ -1106,9 +1108,13 @@ static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedR
     const int tile = MODE == kRowsSwiglu ? kRowsTile : G * kRowsTile;
     const dim3 grid((unsigned)((a.rows + tile - 1) / tile), (unsigned)items);
 #define SB_ROWS(QT)                                                                                       \
-    case QT:                                                                                              \
-        if (pt == 4) launch_kernel(kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a); \
-        else launch_kernel(kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);         \
+    case QT:                                                                                               \
+        if constexpr (G == 1 || (MODE == kRowsSwiglu && QT != QT_Q8_0))                                    \
+            if (pt == 4) {                                                                                 \
+                launch_kernel(kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a);       \
+                break;                                                                                     \
+            }                                                                                              \
+        launch_kernel(kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);               \
         break;
     switch (qt) {
     SB_ROWS(QT_Q8_0)
@@ -1911,7 +1917,7 @@ static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const
                           int n_used, int n_tokens, float* d_out, const float* d_resid, hipStream_t st) {
     if (!rows_layer_ok(L, n_used, n_tokens)) return 1;
     const int run = rows_run(n_used, n_tokens);
-    const int pt = rows_tiles((size_t)run * n_used, L->n_experts, L->d_ff);
+    const int pt = rows_tiles((size_t)run * n_used, L->n_experts, L->d_ff, L->qt_gate == QT_Q8_0);
     if (!grouped_layer_ready(L, n_used, run, pt, st)) return 1;
     for (int t = 0; t < n_tokens; t += run) {
         const size_t td = (size_t)t * L->d_model, tk = (size_t)t * n_used;
@@ -2192,6 +2198,18 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
     return ck(hipGetLastError(), "grouped layer launch") ? 0 : -1;
 }
 
+// The layers the fixed-shape kernels leave to k_grouped_rows: it decodes a row
+// once for up to 64 pairs, where they decode it per 16 (Q4_K, Q6_K) or hold it
+// decoded (IQ3_S gate/up).  Measured (fixed-shape / rows, us; 2048 / 768): Q4_K / Q6_K top-10
+// of 512 446 / 449 at 5 pairs per expert, 502 / 466 at 10, 822 / 578 at 20; top-8 of
+// 128 131 / 135 at 6, 190 / 159 at 16, 795 / 500 at 125; Q4_K / IQ3_S 146 / 150 at
+// 16, 214 / 199 at 32; IQ3_S 467 / 507 at 10, 683 / 598 at 20, 572 / 528 at 125 of
+// 128; over 8 experts Q4_K / Q6_K 34 / 39 at 128 pairs in all, 65 / 47 at 512, IQ3_S 99 / 114 at 2,048.
+static bool prefill_takes_rows(const sabah_moe_layer_desc* L, size_t pairs) {
+    const bool iq3s = L->qt_gate == QT_IQ3_S || L->qt_down == QT_IQ3_S;
+    return pairs >= (iq3s ? 20 : 10) * (size_t)L->n_experts && pairs >= (iq3s ? 4096u : 512u);
+}
+
 SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const float* d_x, const int32_t* d_ids,
                                       const float* d_w, int n_used, int n_tokens, float* d_out, const float* d_resid,
                                       void* stream) {
@@ -2209,6 +2227,10 @@ SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const f
     if (n_tokens == 0) return 0;
     ++g_layer_calls;
     g_lookups += (unsigned long long)n_tokens * n_used;
+    if (prefill_takes_rows(layer, (size_t)n_tokens * n_used)) {
+        const int rc = moe_layer_rows(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, pick_stream(stream));
+        if (rc <= 0) return rc;
+    }
     return moe_grouped_on(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, 0, pick_stream(stream));
 }
 
