@@ -63,6 +63,13 @@ __device__ inline void pin4(V (&v)[4]) {
 }
 __device__ inline long op_of(uint32_t lo, uint32_t hi) { return (long)((uint64_t)hi << 32 | lo); }
 
+typedef _Float16 v4f16 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+__device__ inline u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+template <typename V>
+__device__ inline uint32_t as_word(V v) { return __builtin_bit_cast(uint32_t, v); }
+
 // 256 elements of the lane's row decoded into MFMA B operands (B[s]: lane
 // quarter q's eight elements 32 s + 8 q .. + 7) with the scales of its
 // sub-blocks.  ns: 32-element blocks of the row left (q8_0 formats): the scale
@@ -72,7 +79,7 @@ struct RowOps {
     long B[8];
     uint32_t sc[4];               // packed integer scales (Q8_0, IQ4_NL: none)
     float d[step_q8_0(QT) ? 8 : 2];
-    float mn[2];                  // Q4_K, Q5_K: the mins of items q and q + 4
+    v4f16 mn;                     // Q4_K, Q5_K: the mins of 16-element groups 4 q .. 4 q + 3
 };
 
 template <int QT>
@@ -105,8 +112,9 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
         O.sc[0] = s0 & 0x3F3F3F3Fu;
         O.sc[1] = (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
         const uint32_t m0 = s1 & 0x3F3F3F3Fu, m1 = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
-        O.mn[0] = (float)((m0 >> (8 * q)) & 0xFFu);
-        O.mn[1] = (float)((m1 >> (8 * q)) & 0xFFu);
+        const uint32_t mw = (q & 2 ? m1 : m0) >> (16 * (q & 1));
+        const _Float16 ma = (_Float16)(unsigned short)(mw & 0xFFu), mb = (_Float16)(unsigned short)((mw >> 8) & 0xFFu);
+        O.mn = v4f16{ma, ma, mb, mb};
         O.d[0] = h2f(dd);
         O.d[1] = h2f(dd >> 16);
         const uint64_t qh = QT == QT_Q5_K ? lds_u64x(unit + 16 + 8 * q) : 0;
@@ -165,13 +173,24 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
     }
 }
 
+// two int16 -> two fp16 (exact up to 2,048)
+__device__ inline uint32_t half2_of(uint32_t v) {
+    typedef _Float16 v2f16 __attribute__((ext_vector_type(2)));
+    return as_word(v2f16{(_Float16)(short)(v & 0xFFFFu), (_Float16)(short)(v >> 16)});
+}
+// sum mn_j bs_j over a step's sixteen 16-element groups on fp16 MFMA: exact (the
+// mins are below 64, the sums at most 2,032, every partial sum an integer below 2^24)
+__device__ inline v4f32 min_sums(const v4f16& mn, const v4f16& bs) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(bs, mn, v4f32{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+}
+
 // acc[i] (the lane's row, pair 4 q + i of a tile) += the step's term(s), the
 // unit dot's integers and fp32 steps in its order.  dx: the tile's activation
 // scales (dx[4 q + i]; q8_0: a row of them per 32 elements, dx_stride apart);
-// bs: Q4_K, Q5_K: this lane's two item sums.
+// bs: Q4_K, Q5_K: the 16-element sums 4 q .. 4 q + 3 of pair r.
 template <int QT>
 __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const float* dx, int dx_stride,
-                                 const float (&bs)[2], int q, float (&acc)[4]) {
+                                 const v4f16& bs, int q, float (&acc)[4]) {
     const v4i32 z = {0, 0, 0, 0};
     if constexpr (step_q8_0(QT)) {
 #pragma unroll
@@ -225,10 +244,7 @@ __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const 
             }
         }
         if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
-            // sum mn_j bs_j on fp32 MFMA: exact, every partial sum an integer below 2^24
-            v4f32 ms = {0.0f, 0.0f, 0.0f, 0.0f};
-            ms = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[0], O.mn[0], ms, 0, 0, 0);
-            ms = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[1], O.mn[1], ms, 0, 0, 0);
+            const v4f32 ms = min_sums(O.mn, bs);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 acc[i] = __fadd_rn(acc[i], __fsub_rn(__fmul_rn(__fmul_rn(O.d[0], dxv[i]), (float)isum[i]),
@@ -241,6 +257,90 @@ __device__ inline void step_term(const RowOps<QT>& O, const long (&X)[8], const 
                 acc[i] = __fadd_rn(acc[i], c);
             }
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Four-tile items of Q4_K and Q6_K: the integer scale folded into the weights
+// once, as two int8 operands: scale * q = (hi << SHIFT) + lo.  A step's block sum is
+// then two chains of v_mfma_i32_16x16x64_i8 (64 elements each, the lane's 16
+// bytes of a row's chunk as they lie) that accumulate in the matrix unit, with no
+// multiply-add per 32 elements; the sums are the same exact integers.
+//   Q4_K: q <= 15, sc = 8 a + b: hi = q a, lo = q b, both <= 105 (SHIFT 3);
+//   Q6_K: p = sc (q - 32), |p| <= 4,096: hi = p >> 7 (-32 .. 32), lo = p & 127 (SHIFT 7).
+// ---------------------------------------------------------------------------
+template <int QT>
+struct FoldOps {
+    v4i32 hi[4], lo[4];
+    float d[2];
+    v4f16 mn;
+};
+template <int QT>
+__device__ inline void fold_ops(const uint8_t* unit, int q, FoldOps<QT>& F) {
+    if constexpr (QT == QT_Q4_K) {
+        RowOps<QT> O;
+        row_ops<QT>(unit, nullptr, q, 8, O);
+        F.d[0] = O.d[0];
+        F.d[1] = O.d[1];
+        F.mn = O.mn;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t sc = (O.sc[s >> 2] >> (8 * (s & 3))) & 0xFFu;
+            const unsigned short b = (unsigned short)(sc & 7u), a = (unsigned short)(sc >> 3);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const u16x2 w = as_u16x2((uint32_t)((uint64_t)O.B[s] >> (32 * u)));   // bytes <= 15: no carry into the next
+                F.hi[s >> 1][2 * (s & 1) + u] = (int)as_word(w * u16x2{a, a});
+                F.lo[s >> 1][2 * (s & 1) + u] = (int)as_word(w * u16x2{b, b});
+            }
+        }
+    } else {
+        static_assert(QT == QT_Q6_K, "folded formats: Q4_K, Q6_K");
+        F.d[0] = h2f(lds_u16(unit + 208));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint64_t l0 = lds_u64f(unit + 64 * h + 8 * q), l1 = lds_u64f(unit + 64 * h + 32 + 8 * q);
+            const uint64_t hb = lds_u64f(unit + 128 + 32 * h + 8 * q), sw = lds_u64f(unit + 192 + 8 * h);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int s = 4 * h + t;
+                const uint64_t lo = (t & 1 ? l1 : l0) >> (4 * (t >> 1)), hi = hb >> (2 * t);
+                const uint64_t v = (lo & 0x0F0F0F0F0F0F0F0Full) | ((hi & 0x0303030303030303ull) << 4);
+                // the lane's elements lie in half q / 2 of the item: scale byte 2 t + q / 2
+                const int sc = (int)(int8_t)((uint32_t)(sw >> (32 * (t >> 1))) >> (16 * (t & 1) + 8 * (q >> 1)));
+                const unsigned short m16 = (unsigned short)sc, c16 = (unsigned short)(-32 * sc);
+                const u16x2 m = {m16, m16}, c = {c16, c16};
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const uint32_t w = (uint32_t)(v >> (32 * u));
+                    const u16x2 pe = as_u16x2(w & 0x00FF00FFu) * m + c, po = as_u16x2((w >> 8) & 0x00FF00FFu) * m + c;
+                    const uint32_t he = as_word(__builtin_bit_cast(i16x2, pe) >> 7), ho = as_word(__builtin_bit_cast(i16x2, po) >> 7);
+                    F.hi[s >> 1][2 * (s & 1) + u] = (int)__builtin_amdgcn_perm(ho, he, 0x06020400u);
+                    F.lo[s >> 1][2 * (s & 1) + u] = (int)((as_word(pe) & 0x007F007Fu) | (as_word(po) & 0x007F007Fu) << 8);
+                }
+            }
+        }
+    }
+}
+template <int QT>
+__device__ inline void fold_term(const FoldOps<QT>& F, const v4i32 (&X)[4], const float* dx, const v4f16& bs, int q,
+                                 float (&acc)[4]) {
+    v4i32 H = {0, 0, 0, 0}, L = {0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        H = __builtin_amdgcn_mfma_i32_16x16x64_i8(X[t], F.hi[t], H, 0, 0, 0);
+        L = __builtin_amdgcn_mfma_i32_16x16x64_i8(X[t], F.lo[t], L, 0, 0, 0);
+    }
+    const float4 dx4 = *reinterpret_cast<const float4*>(dx + 4 * q);
+    const float dxv[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+    v4f32 ms = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (QT == QT_Q4_K) ms = min_sums(F.mn, bs);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int isum = H[i] * (QT == QT_Q4_K ? 8 : 128) + L[i];
+        float c = __fmul_rn(__fmul_rn(F.d[0], dxv[i]), (float)isum);
+        if constexpr (QT == QT_Q4_K) c = __fsub_rn(c, __fmul_rn(__fmul_rn(F.d[1], dxv[i]), ms[i]));
+        acc[i] = __fadd_rn(acc[i], c);
     }
 }
 
@@ -271,6 +371,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a)
     constexpr int NT = kThreads, CB = step_bytes(QT), CPR = step_chunks(QT);
     constexpr int NLM = (kRowsTile * CPR + NT - 1) / NT, NL = G * NLM, TP = 16 * PT;   // loads per row group and in all
     constexpr bool Q80 = step_q8_0(QT), BS = QT == QT_Q4_K || QT == QT_Q5_K;
+    constexpr bool FOLD = PT == 4 && (QT == QT_Q4_K || QT == QT_Q6_K);
     // a row's address mod 16 is the same at every step
     constexpr bool FIXED = CB % 16 == 0;
     typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
@@ -278,7 +379,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a)
     __shared__ __align__(16) uint8_t raw[NL * NT * 16 + 16];   // 16: dwords read past a field's end
     __shared__ __align__(16) uint8_t xs[TP * kActChunkStride];
     __shared__ __align__(16) float sdx[(Q80 ? 8 : 1) * TP];
-    __shared__ __align__(16) float sbs[BS ? TP * 8 : 4];
+    __shared__ __align__(16) uint32_t sbs[BS ? TP * 8 : 4];  // 16 fp16 sums per pair
     __shared__ size_t sdst[MMID ? TP : 1];                   // byte offset of each pair's dst row
     const int4 it = a.items[blockIdx.y];
     if ((int)blockIdx.y >= *a.n_items) return;               // uniform: the list is shorter than its bound
@@ -375,6 +476,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a)
 #pragma unroll
     for (int m = 0; m < G; ++m) my_row[m] = (uint32_t)row_of(m, 16 * wave + r) * (uint32_t)rb;
     const uint8_t* const xl = xs + r * kActChunkStride + 16 * q;
+    // the lane's staged row of group m at step s
+    auto unit_of = [&](int m, int s) {
+        const uint32_t lead = ((uint32_t)reinterpret_cast<uintptr_t>(base[m]) + my_row[m] + (uint32_t)(s * CB)) & 15u;
+        return raw + NLM * NT * 16 * m + (16 * wave + r) * (16 * CPR) + lead;
+    };
     auto read_x = [&](int p, long (&X)[8]) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -394,33 +500,48 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_rows(GroupedRowsArgs a)
             *reinterpret_cast<u32x4*>(xs + (16 * p + xp) * kActChunkStride + 16 * xk) = xd[p];
             if (Q80 ? xk < 8 : xk == 0) sdx[(Q80 ? TP * xk : 0) + 16 * p + xp] = xdx[p];
             if (BS && xk < 8)
-                sbs[8 * (16 * p + xp) + xk] = (float)((int)(int16_t)(xbs[p] & 0xFFFFu) + ((int)xbs[p] >> 16));
+                sbs[8 * (16 * p + xp) + xk] = half2_of(xbs[p]);
         }
         __syncthreads();
         if (s + 1 < nch) {
             load_w(s + 1);
             load_xs(s + 1);
         }
-        const int ns = Q80 ? (a.k - 256 * s) >> 5 : 8;
-        long X[8];
-        read_x(0, X);
-        RowOps<QT> O[G];
+        if constexpr (FOLD) {
+            // one group at a time: its operands take 32 registers
 #pragma unroll
-        for (int m = 0; m < G; ++m) {
-            const uint32_t lead = ((uint32_t)reinterpret_cast<uintptr_t>(base[m]) + my_row[m] + (uint32_t)(s * CB)) & 15u;
-            row_ops<QT>(raw + NLM * NT * 16 * m + (16 * wave + r) * (16 * CPR) + lead, tabs, q, ns, O[m]);
-        }
+            for (int m = 0; m < G; ++m) {
+                FoldOps<QT> F;
+                fold_ops<QT>(unit_of(m, s), q, F);
 #pragma unroll
-        for (int p = 0; p < PT; ++p) {
-            if (p >= nt) continue;
-            if (p) read_x(p, X);
-            float bs[2] = {0.0f, 0.0f};
-            if constexpr (BS) {
-                bs[0] = sbs[8 * (16 * p + r) + q];
-                bs[1] = sbs[8 * (16 * p + r) + q + 4];
+                for (int p = 0; p < PT; ++p) {
+                    if (p >= nt) continue;
+                    v4i32 X[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) X[t] = *reinterpret_cast<const v4i32*>(xl + 16 * p * kActChunkStride + 64 * t);
+                    v4f16 bs = {0, 0, 0, 0};
+                    if constexpr (BS) bs = *reinterpret_cast<const v4f16*>(sbs + 8 * (16 * p + r) + 2 * q);
+                    fold_term<QT>(F, X, sdx + 16 * p, bs, q, acc[m][p]);
+                }
+            }
+        } else {
+            const int ns = Q80 ? (a.k - 256 * s) >> 5 : 8;
+            long X[8];
+            read_x(0, X);
+            RowOps<QT> O[G];
+#pragma unroll
+            for (int m = 0; m < G; ++m) {
+                row_ops<QT>(unit_of(m, s), tabs, q, ns, O[m]);
             }
 #pragma unroll
-            for (int m = 0; m < G; ++m) step_term<QT>(O[m], X, sdx + 16 * p, TP, bs, q, acc[m][p]);
+            for (int p = 0; p < PT; ++p) {
+                if (p >= nt) continue;
+                if (p) read_x(p, X);
+                v4f16 bs = {0, 0, 0, 0};
+                if constexpr (BS) bs = *reinterpret_cast<const v4f16*>(sbs + 8 * (16 * p + r) + 2 * q);
+#pragma unroll
+                for (int m = 0; m < G; ++m) step_term<QT>(O[m], X, sdx + 16 * p, TP, bs, q, acc[m][p]);
+            }
         }
     }
 #pragma unroll
