@@ -89,8 +89,18 @@ __device__ inline uint32_t low_bytes4(uint32_t a, uint32_t b, uint32_t c, uint32
 // grouped kernels' operand order, in which the element k = 32 s + 8 q + i
 // (sub-block s, quarter q, i < 8) sits at byte 64 (s / 2) + 16 q + 8 (s % 2) + i,
 // so one 16-byte load gives an MFMA lane its eight elements of two
-// sub-blocks.
-__device__ inline void mfma_chunk_store(uint8_t* chunk, uint32_t l, const uint4& packed) {
+// sub-blocks.  Order 2, for the formats whose 16 bytes per sub-block hold
+// elements i and 16 + i in a byte: quarter q's eight are 4 q .. 4 q + 3 and 16 + 4 q
+// .. + 3, so a lane's eight weights are the two nibbles of one dword.
+__device__ inline void mfma_chunk_store(uint8_t* chunk, uint32_t l, const uint4& packed, int order) {
+    if (order == 2) {
+        uint32_t* o = reinterpret_cast<uint32_t*>(chunk + 64 * (l >> 2) + 8 * ((l >> 1) & 1u) + 4 * (l & 1u));
+        o[0] = packed.x;
+        o[4] = packed.y;
+        o[8] = packed.z;
+        o[12] = packed.w;
+        return;
+    }
     // quarters 2 (l & 1) and 2 (l & 1) + 1 of sub-block l / 2
     uint8_t* o = chunk + 64 * (l >> 2) + 32 * (l & 1u) + 8 * ((l >> 1) & 1u);
     *reinterpret_cast<uint2*>(o) = make_uint2(packed.x, packed.y);
@@ -107,7 +117,7 @@ __device__ inline void mfma_chunk_store(uint8_t* chunk, uint32_t l, const uint4&
 // rounds to at most 127, so ggml's clamp at 127 never applies.
 // mfma_order: the chunk's 256 bytes in the grouped kernels' operand order
 // (mfma_chunk_store; bsums and d unchanged).
-__device__ inline void row16_quant_q8K(const Act16& a, int c, uint8_t* act, const ActLayout& L, bool mfma_order = false) {
+__device__ inline void row16_quant_q8K(const Act16& a, int c, uint8_t* act, const ActLayout& L, int mfma_order = 0) {
     const uint32_t l = threadIdx.x & 15u;
     float mx_l = a.v[0], mn_l = a.v[0];
 #pragma unroll
@@ -142,7 +152,7 @@ __device__ inline void row16_quant_q8K(const Act16& a, int c, uint8_t* act, cons
     packed.y = low_bytes4(b[4], b[5], b[6], b[7]);
     packed.z = low_bytes4(b[8], b[9], b[10], b[11]);
     packed.w = low_bytes4(b[12], b[13], b[14], b[15]);
-    if (mfma_order) mfma_chunk_store(act + c * kActChunkStride, l, packed);
+    if (mfma_order) mfma_chunk_store(act + c * kActChunkStride, l, packed, mfma_order);
     else reinterpret_cast<uint4*>(act + c * kActChunkStride)[l] = packed;
     // bsum = sum of the sixteen int8 values
     int s = 0;
@@ -158,7 +168,7 @@ __device__ inline void row16_quant_q8K(const Act16& a, int c, uint8_t* act, cons
 // (with_sum) also stores s = fp16(sum(q) * d), d the fp32 scale before its
 // fp16 rounding (quantize_row_q8_1_ref), in the layout's s area.
 __device__ inline void row16_quant_q8_0(const Act16& a, int c, uint8_t* act, const ActLayout& L,
-                                        bool with_sum = false, bool mfma_order = false) {
+                                        bool with_sum = false, int mfma_order = 0) {
     const uint32_t l = threadIdx.x & 15u;
     float amax = 0.0f;
 #pragma unroll
@@ -174,7 +184,7 @@ __device__ inline void row16_quant_q8_0(const Act16& a, int c, uint8_t* act, con
     packed.y = pack4_i8(q[4], q[5], q[6], q[7]);
     packed.z = pack4_i8(q[8], q[9], q[10], q[11]);
     packed.w = pack4_i8(q[12], q[13], q[14], q[15]);
-    if (mfma_order) mfma_chunk_store(act + c * kActChunkStride, l, packed);
+    if (mfma_order) mfma_chunk_store(act + c * kActChunkStride, l, packed, mfma_order);
     else reinterpret_cast<uint4*>(act + c * kActChunkStride)[l] = packed;
     if ((l & 1u) == 0) reinterpret_cast<float*>(act + L.off_d)[c * 8 + (l >> 1)] = __half2float(__float2half_rn(d));
     if (with_sum) {
@@ -255,7 +265,7 @@ __device__ inline void act_prefetch(const ActBatch& B, ActRegs<ROUNDS>& R, int w
     }
 }
 
-__device__ inline void quant_chunk(const ActBatch& B, const Act16& a_in, int q, bool mfma_order = false) {
+__device__ inline void quant_chunk(const ActBatch& B, const Act16& a_in, int q, int mfma_order = 0) {
     const int nch = (B.k + 255) / 256;
     const int r = div_small(q, __builtin_amdgcn_rcpf((float)nch)), c = q - r * nch;
     const ActLayout L(B.k, B.at);

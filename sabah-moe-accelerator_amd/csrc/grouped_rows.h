@@ -32,6 +32,9 @@ __host__ __device__ constexpr bool grouped_rows_type(int qt) {
            qt == QT_IQ4_NL || qt == QT_IQ4_XS;
 }
 
+// the order of the activations' bytes (mfma_chunk_store)
+__host__ __device__ constexpr int rows_act_order(int qt) { return qt == QT_IQ4_NL || qt == QT_IQ4_XS ? 2 : 1; }
+
 // reads at any even LDS address
 struct __attribute__((packed, aligned(2))) LdsU32x {
     uint32_t v;
@@ -71,7 +74,7 @@ template <typename V>
 __device__ inline uint32_t as_word(V v) { return __builtin_bit_cast(uint32_t, v); }
 
 // 256 elements of the lane's row decoded into MFMA B operands (B[s]: lane
-// quarter q's eight elements 32 s + 8 q .. + 7) with the scales of its
+// quarter q's eight elements 32 s + 8 q .. + 7, or of mfma_chunk_store's order 2) with the scales of its
 // sub-blocks.  ns: 32-element blocks of the row left (q8_0 formats): the scale
 // of a block past the row is 0, and so is its term (its activations are zeros).
 template <int QT>
@@ -155,8 +158,8 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
     } else if constexpr (QT == QT_IQ4_NL) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const uint64_t n = (lds_u64f(unit + 18 * s + 2 + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
-            O.B[s] = op_of(iq4_levels((uint32_t)n), iq4_levels((uint32_t)(n >> 32)));
+            const uint32_t n = lds_u32f(unit + 18 * s + 2 + 4 * q);
+            O.B[s] = op_of(iq4_levels(n & 0x0F0F0F0Fu), iq4_levels((n >> 4) & 0x0F0F0F0Fu));
             O.d[s] = s < ns ? h2f(lds_u16(unit + 18 * s)) : 0.0f;
         }
     } else {
@@ -166,8 +169,8 @@ __device__ inline void row_ops(const uint8_t* unit, const uint8_t* tabs, int q, 
         O.sc[0] = O.sc[1] = 0;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const uint64_t n = (lds_u64x(unit + 8 + 16 * s + 8 * (q & 1)) >> (4 * (q >> 1))) & 0x0F0F0F0F0F0F0F0Full;
-            O.B[s] = op_of(iq4_levels((uint32_t)n), iq4_levels((uint32_t)(n >> 32)));
+            const uint32_t n = lds_u32x(unit + 8 + 16 * s + 4 * q);
+            O.B[s] = op_of(iq4_levels(n & 0x0F0F0F0Fu), iq4_levels((n >> 4) & 0x0F0F0F0Fu));
             O.sc[s >> 2] |= (((sl >> (4 * s)) & 15u) | (((sh >> (2 * s)) & 3u) << 4)) << (8 * (s & 3));
         }
     }

@@ -89,8 +89,8 @@ __device__ inline int block_exclusive_scan(int v, int* tmp, int& total) {
 }
 
 // ids a thread keeps in registers between the histogram and the scatter
-// (n_tokens * k up to 8 x 1024); larger batches re-read them
-constexpr int kGroupIdRegs = 8;
+// (n_tokens * k up to 16 x 1024); larger batches re-read them
+constexpr int kGroupIdRegs = 16;
 
 // one workgroup of kGroupThreads; dynamic LDS: 2 * n_experts + kGroupThreads ints
 __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
 // floats.  Each workgroup quantises 16 chunk-rows (one per 16-lane row).
 // With `gather`, output row r is input row gather[r] / gdiv, for the rows
 // below *count (the grouped pairs: the rows come out in group order).  With
-// mfma_order (q8_K, q8_0), each chunk's bytes are in the grouped kernels'
+// mfma_order 1 or 2 (q8_K, q8_0), each chunk's bytes are in the grouped kernels'
 // operand order (mfma_chunk_store).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void k_quant_rows(const float* __restrict__ x, int n_rows, int k, int at,
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kThreads) void k_quant_rows(const float* __restrict
     const ActBatch B{x, (size_t)k, n_rows, k, at, out, out_stride};
     Act16 v;
     load16(x + (size_t)src * k, c * 256 + 16 * (int)(threadIdx.x & 15u), k, act_vec(B), v);
-    quant_chunk(B, v, q, mfma_order != 0);
+    quant_chunk(B, v, q, mfma_order);
 }
 
 // ---------------------------------------------------------------------------

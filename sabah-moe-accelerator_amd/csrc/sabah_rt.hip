@@ -1093,7 +1093,7 @@ static void launch_quant_mfma(int kind, const float* x, size_t n, int k, int qt,
                               const int* count, hipStream_t st) {
     const size_t chunks = n * (size_t)((k + 255) / 256);
     launch_kernel(kind, k_quant_rows, dim3((unsigned)((chunks + 15) / 16)), dim3(kThreads), 0, st, x, (int)n, k,
-                  act_type(qt), out, stride, (const int*)nullptr, 1, count, 1);
+                  act_type(qt), out, stride, (const int*)nullptr, 1, count, rows_act_order(qt));
 }
 // Two 16-row groups per wave (128-row tiles, the activations read from LDS
 // once for both) for two-tile items, where 128-row tiles fit the rows and the launch
