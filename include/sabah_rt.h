@@ -285,7 +285,7 @@ int sabah_moe_route(const float *d_logits, int n_tokens, int n_experts, int n_us
  * eligible calls have packed rows, dense ids and x, n_experts <= 4096 and a
  * type of Q8_0, Q4_K, Q5_K, Q6_K, IQ3_S, IQ3_XXS, IQ4_NL or IQ4_XS.
  * mode 0 (default): grouped when eligible with enough pairs per expert on
- * average (1 or 2, by type and shape); 1: never; 2: whenever eligible.
+ * average (by type and shape); 1: never; 2: whenever eligible.
  * The results are bit-identical either way.  IQ3_S, Q4_K and Q6_K calls with
  * k <= 1024, k % 256 == 0 and rows % 64 == 0, or k % 512 == 0, k <= 2048 and rows % 32
  * == 0, use library scratch (pair lists, q8 rows) shared by every stream when

@@ -1135,18 +1135,35 @@ static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRow
     else launch_rows_g<1, MODE>(qt, kind, pt, items, a, st);
 }
 
-// The general grouped form needs at least this many pairs per expert on
-// average, and kRowsMinPairs in all.  Measured (token-major / grouped, us):
-// one layer, top-10 of 512, 2048 / 768: IQ4_XS 178 / 154 at 0.31 pairs per expert,
-// Q5_K 217 / 217 and IQ3_XXS / IQ4_NL 269 / 247 at 0.62, Q8_0 625 / 543 and
-// IQ3_S 336 / 377 at 1.25; top-8 of 128 Q8_0 126 / 144 at 1, 247 / 196 at 2; gate and down
-// nodes cross at the same densities.  Below kRowsMinPairs the grouping's own
-// launches decide: top-2 of 8, 1024 / 2048, a Q8_0 layer 33 / 47 at 16 pairs, 51 / 47 at 32
-// and 158 / 54 at 128, a gate node 17 / 18 at 32 and 55 / 20 at 128.
-constexpr long long kRowsMinPairs = 64;
-static int rows_min_pairs(int qt) { return qt == QT_IQ4_XS || qt == QT_Q5_K || qt == QT_IQ3_XXS ? 1 : 2; }
-static bool rows_worth_it(int qt, long long pairs, int n_experts) {
-    return pairs >= kRowsMinPairs && pairs >= (long long)rows_min_pairs(qt) * n_experts;
+// Where the general grouped form is the faster one: from base pairs (for
+// matrices of 2 M weights; the grouping's own launches, so in inverse proportion to the
+// matrix) plus per16 / 16 for every expert (whose rows it reads once, where the token-major
+// kernels read them for each pair).  Measured crossings, in pairs, at 512 / 128 / 64 / 8
+// experts (2048 / 768, IQ3_XXS and IQ4_NL 2560 / 640; 8 experts 1024 / 2048):
+//   layer    Q8_0 and Q6_K gate/up 180 / 100 / 64 / 24, Q4_K 440 / 145 / 96 / 28, Q5_K 230 / 105 / 65 / 22, IQ3_S
+//            900 / 260 / 150 / 44, IQ3_XXS 200 / 136 / 112 / 48, IQ4_XS 100 / 80 / 65 / 24
+//   MUL_MAT_ID  Q8_0 gate 205 / 125 / 75 / 32, down 485 / 150 / 100 / 36; Q5_K 360 - 480 / 130 - 150 / 85 - 110 / 36;
+//            IQ4_XS 130 - 230 / 110 - 140 / 85 - 130 / 32; IQ3_XXS gate 290 / 170 / 130 / 110, IQ4_NL down 970 / 245 / 145 / 56
+// e.g. (token-major / grouped, us) an IQ4_XS layer at 32 tokens, top-10 of 512: 374 / 218; Q8_0
+// at 16 tokens, top-2 of 8: 51 / 41, at 8: 32 / 41.
+struct RowsCost {
+    int base, per16;
+};
+static RowsCost rows_cost(int qt, bool layer) {
+    switch (qt) {
+    case QT_Q8_0: return layer ? RowsCost{24, 9} : RowsCost{36, 14};
+    case QT_Q6_K: return layer ? RowsCost{24, 9} : RowsCost{36, 12};
+    case QT_Q4_K: return layer ? RowsCost{28, 16} : RowsCost{48, 18};
+    case QT_Q5_K: return layer ? RowsCost{24, 10} : RowsCost{36, 14};
+    case QT_IQ3_S: return layer ? RowsCost{44, 28} : RowsCost{60, 24};
+    case QT_IQ3_XXS: return layer ? RowsCost{40, 11} : RowsCost{80, 10};
+    case QT_IQ4_XS: return layer ? RowsCost{32, 7} : RowsCost{36, 9};
+    default: return layer ? RowsCost{44, 28} : RowsCost{44, 29};       // IQ4_NL
+    }
+}
+static bool rows_worth_it(int qt, bool layer, size_t pairs, int n_experts, int rows, int k) {
+    const RowsCost c = rows_cost(qt, layer);
+    return 16.0 * (double)pairs >= 16.0 * c.base * (double)(1 << 21) / ((double)rows * k) + (double)c.per16 * n_experts;
 }
 static bool mmid_rows_ok(int qt, bool packed, const uint8_t* bank, size_t expert_stride, size_t ids_id_stride,
                          size_t ids_token_stride, size_t x_id_stride, size_t x_token_stride, int x_rows, int n_ids,
@@ -1371,7 +1388,7 @@ SABAH_API int sabah_rt_mul_mat_id_v2(const void* source, size_t expert_stride, s
                 return -1;
             grouped = true;
         }
-    } else if (mode != 1 && (mode == 2 || rows_worth_it(qt, pairs, n_experts)) &&
+    } else if (mode != 1 && (mode == 2 || rows_worth_it(qt, false, (size_t)pairs, n_experts, rows, k)) &&
                mmid_rows_ok(qt, packed, bank, expert_stride, ids_id_stride, ids_token_stride, x_id_stride,
                             x_token_stride, x_rows, n_ids, n_tokens, rows, k, n_experts)) {
         const int rc = mmid_rows(qt, bank, expert_stride, static_cast<const float*>(d_x), x_rows,
@@ -1903,7 +1920,7 @@ constexpr size_t kRowsMaxPairs = 65536;
 static int rows_run(int n_used, int n_tokens) { return std::min(n_tokens, std::max(1, (int)(kRowsMaxPairs / n_used))); }
 static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
     const size_t P = (size_t)rows_run(n_used, n_tokens) * n_used;
-    return n_tokens >= 2 && rows_worth_it(L->qt_gate, (long long)P, L->n_experts) &&
+    return n_tokens >= 2 && rows_worth_it(L->qt_gate, true, P, L->n_experts, L->d_ff, L->d_model) &&
            rows_shape_ok(L->qt_gate, P, L->n_experts, L->d_ff, L->d_model) &&
            rows_shape_ok(L->qt_down, P, L->n_experts, L->d_model, L->d_ff) &&
            rows_bank_ok(L->gate, row_bytes(L->qt_gate, L->d_model) * L->d_ff) && rows_bank_ok(L->up, 0) &&

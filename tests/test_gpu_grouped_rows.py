@@ -117,7 +117,7 @@ def test_a_bad_id_becomes_nan_and_is_reported(hip_rt, grouping):
 def test_calls_on_two_streams_and_under_capture(hip_rt, grouping):
     """Two streams' calls overlap with workspaces of their own, and a captured
     call (token-major) replays beside them."""
-    E, K, rows, k, tokens = 7, 2, 96, 768, 200
+    E, K, rows, k, tokens = 7, 2, 960, 768, 200
     rng = np.random.default_rng(6)
     bank = T(bank_bytes(rng, IQ3_XXS, E, rows, k))
     xs = [T(rng.standard_normal((tokens, 1, k)).astype(np.float32)) for _ in range(2)]
@@ -155,6 +155,13 @@ def test_calls_on_two_streams_and_under_capture(hip_rt, grouping):
     assert hip_rt.snapshot()["grouped_calls"] == before + 20
 
 
+def grouped_launches(hip_rt):
+    """Group-major gate/up launches (kernel kind 4) since the last reading, with timing on."""
+    ms, n = ctypes.c_double(), ctypes.c_ulonglong()
+    hip_rt.check(hip_rt.lib().sabah_rt_get_kernel_timing(4, ctypes.byref(ms), ctypes.byref(n), 1), "timing")
+    return n.value
+
+
 def layer(hip_rt, fn, desc, x, ids, w, resid=None):
     out = torch.full_like(x, float("nan"))
     hip_rt.check(getattr(hip_rt.lib(), fn)(
@@ -164,10 +171,14 @@ def layer(hip_rt, fn, desc, x, ids, w, resid=None):
     return out.cpu().numpy()
 
 
-@pytest.mark.parametrize("qtg,qtd,D,F", [(IQ3_XXS, IQ4_NL, 2560, 640), (Q8_0, Q8_0, 288, 96), (Q5_K, IQ4_XS, 512, 256),
-                                         (Q4_K, Q6_K, 256, 1280), (Q6_K, Q8_0, 768, 352), (IQ3_S, IQ3_S, 512, 512),
-                                         (IQ3_XXS, IQ4_NL, 16640, 64)])
-@pytest.mark.parametrize("tokens", [33, 61])
+# the tokens are the fewest that take the grouped form at the shape, and more; 16640 rows give
+# each wave of the down kernel two row groups
+LAYERS = [(IQ3_XXS, IQ4_NL, 2560, 640, (28, 61)), (Q8_0, Q8_0, 288, 96, (912, 1001)), (Q5_K, IQ4_XS, 512, 256, (194, 301)),
+          (Q4_K, Q6_K, 256, 1280, (93, 150)), (Q6_K, Q8_0, 768, 352, (95, 150)), (IQ3_S, IQ3_S, 512, 512, (182, 301)),
+          (IQ3_XXS, IQ4_NL, 16640, 64, (42, 61))]
+
+
+@pytest.mark.parametrize("qtg,qtd,D,F,tokens", [(*c[:4], t) for c in LAYERS for t in c[4]])
 def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, tokens):
     from sabah.runtime import rt
     E, K = 6, 2
@@ -183,7 +194,12 @@ def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, t
     w = T(rng.random((tokens, K)).astype(np.float32))
     for resid in (None, T(rng.standard_normal((tokens, D)).astype(np.float32))):
         want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x, ids, w, resid)
-        assert_bits_equal(layer(hip_rt, "sabah_moe_layer", desc, x, ids, w, resid), want, "layer")
+        hip_rt.check(hip_rt.lib().sabah_rt_set_kernel_timing(1), "timing on")
+        grouped_launches(hip_rt)
+        got = layer(hip_rt, "sabah_moe_layer", desc, x, ids, w, resid)
+        assert grouped_launches(hip_rt) > 0
+        hip_rt.check(hip_rt.lib().sabah_rt_set_kernel_timing(0), "timing off")
+        assert_bits_equal(got, want, "layer")
     # in place, then captured with the scratch in place
     y = x.clone()
     graph = torch.cuda.CUDAGraph()
