@@ -105,7 +105,8 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
 #pragma unroll
     for (int i = 0; i < kGroupIdRegs; ++i) {
         const int p = tid + NT * i;
-        idv[i] = in_regs && p < P ? a.ids[p] : -1;
+        idv[i] = -1;
+        if (in_regs && NT * i < P) idv[i] = a.ids[min(p, P - 1)];      // uniform
     }
     for (int e = tid; e < E; e += NT) cnt[e] = 0;
     __syncthreads();
@@ -113,8 +114,10 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_pairs(GroupArgs a) {
     auto each_pair = [&](auto&& f) {
         if (in_regs) {
 #pragma unroll
-            for (int i = 0; i < kGroupIdRegs; ++i)
+            for (int i = 0; i < kGroupIdRegs; ++i) {
+                if (NT * i >= P) break;                     // uniform: a small batch skips the rest
                 if (tid + NT * i < P) f(tid + NT * i, idv[i]);
+            }
         } else {
             for (int p = tid; p < P; p += NT) f(p, a.ids[p]);
         }

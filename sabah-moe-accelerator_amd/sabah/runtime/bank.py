@@ -138,10 +138,10 @@ class ExpertBank:
 
     def layer_desc(self, layer: int, shared=None) -> rt.MoeLayerDesc:
         """sabah_moe_layer_desc of one layer; shared = DenseExpert or None."""
-        d = rt.MoeLayerDesc()
-        d.gate, d.up, d.down = (self.base_ptr(layer, r) for r in ROLES)
-        d.qt_gate, d.qt_up, d.qt_down = (self.lq[(layer, r)] for r in ROLES)
-        d.d_model, d.d_ff, d.n_experts = self.d_model, self.d_ff, self.n_experts
+        base, off, lq = self.storage.data_ptr(), self.offsets, self.lq
+        g, u, n = (layer, "gate"), (layer, "up"), (layer, "down")
+        d = rt.MoeLayerDesc(base + off[g], base + off[u], base + off[n], lq[g], lq[u], lq[n],
+                            self.d_model, self.d_ff, self.n_experts)
         if shared is not None:
             d.shared_gate, d.shared_up, d.shared_down = shared.ptrs()
             d.qt_shared_gate = d.qt_shared_up = d.qt_shared_down = shared.qt

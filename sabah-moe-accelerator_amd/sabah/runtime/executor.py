@@ -28,12 +28,17 @@ from . import rt
 from .bank import ROLES, DenseExpert, ExpertBank
 
 
-def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# A small call is bound by what Python does before the launch, so the hot
+# methods read each tensor's strides once and pass plain integers where the
+# binding declares pointers.  Measured on an eager Q4_K gate node, one token (kernel 5 us):
+# 9.7 us a call before, 7.2 after; the router at 8 tokens 8.9, 7.6.
+def _stream(device) -> int:
+    """The handle of torch's current stream on the device (no Stream object made)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
-def _vp(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _vp(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 class MoEExecutor:
@@ -103,15 +108,19 @@ class MoEExecutor:
         T, n_ids = ids.shape
         rows, k, qt = b.rows[role], b.cols[role], b.layer_qtype(layer, role)
         if out is None:
-            out = torch.empty(T, n_ids, rows, dtype=torch.float32, device=self.device)
+            out = torch.empty((T, n_ids, rows), dtype=torch.float32, device=self.device)
         src = b.base_ptr(layer, role) if source is None else source
+        row_bytes = rt.row_bytes(qt, k)
+        xs, ns, os = x.stride(), ids.stride(), out.stride()
+        ids_ptr = ids.data_ptr()
         rc = rt.lib().sabah_rt_mul_mat_id_v2(
-            ctypes.c_void_p(src), b.layer_stride(layer, role), b.layer_row_bytes(layer, role),
-            _vp(x), x.stride(1) * 4, x.shape[1], x.stride(0) * 4,
-            _vp(ids), ids.stride(1) * 4, ids.stride(0) * 4, n_ids, T,
-            _vp(out), out.stride(1) * 4, out.stride(0) * 4,
-            rows, k, b.n_experts, qt, _stream(self.device), _vp(ids))
-        rt.check(rc, "MUL_MAT_ID")
+            src, rows * row_bytes, row_bytes,
+            x.data_ptr(), xs[1] * 4, x.shape[1], xs[0] * 4,
+            ids_ptr, ns[1] * 4, ns[0] * 4, n_ids, T,
+            out.data_ptr(), os[1] * 4, os[0] * 4,
+            rows, k, b.n_experts, qt, _stream(self.device), ids_ptr)
+        if rc:
+            rt.check(rc, "MUL_MAT_ID")
         return out
 
     # ---- fused layer / chain --------------------------------------------------
