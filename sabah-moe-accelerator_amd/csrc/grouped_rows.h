@@ -12,6 +12,12 @@
 // MFMA operands for all of the item's 16-pair tiles.  A row's fp32 sum is kept
 // in the lane and grows in block order, so the results are the token-major
 // kernels', bit for bit, in every format.
+//
+// What bounds it: decoding.  A 512-token IQ3_XXS / IQ4_NL layer (top-10 of 512,
+// 2560 / 640; 1.1 GB of weights): gate/up 285 us (2.25 TB/s; VALU busy 67 %, LDS 62 %, most of
+// it codebook look-ups), down 253 us (1.87 TB/s; VALU 63 %, LDS 30 %), two to three waves per
+// SIMD; the layer 516 us against 4,680 token-major.  A Q4_K / Q6_K layer at 1,999 tokens,
+// top-8 of 128 (125 pairs per expert): 432 us against 777 with the fixed-shape kernels.
 #pragma once
 #include "prefill_kernels.h"
 

@@ -1948,12 +1948,14 @@ static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const
 static int moe_layer_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                         int n_used, int n_tokens, float* d_out, const float* d_resid, Workspace& ws, hipStream_t st) {
     const int D = L->d_model, F = L->d_ff;
+    // sized for the token-major form also where the grouped one runs: a smaller call
+    // captured later may take the former, and cannot grow them
+    LayerBufs b;
+    if (layer_bufs(L, n_used, n_tokens, ws, st, b)) return -1;
     if (!ws.arena) {
         const int rc = moe_layer_rows(L, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, st);
         if (rc <= 0) return rc;
     }
-    LayerBufs b;
-    if (layer_bufs(L, n_used, n_tokens, ws, st, b)) return -1;
     std::unique_lock<std::mutex> side_lock(g_side_mu, std::defer_lock);
     hipEvent_t join = nullptr;
     if (shared_overlaps(L, n_tokens)) {
@@ -2079,14 +2081,15 @@ static bool grouped_shape_ok(const sabah_moe_layer_desc* L) {
 
 // Scratch of a group-major layer.  pt = 0: the fixed-shape kernels' (the
 // pairs' x rows quantised in group order); pt = 2, 4: k_grouped_rows with items of pt
-// 16-pair tiles (one q8 row per token, and the item list).
+// 16-pair tiles (one q8 row per token; xq is sized for the pairs all the same,
+// so a smaller call that takes the other kernels finds its room in a capture).
 struct GroupedBufs {
     size_t index, xq, h, hq, y;
 };
 static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt) {
     const size_t P = (size_t)n_tokens * n_used;
     return {rows_index_bytes(P, L->n_experts, pt ? pt : 2),
-            ActLayout(L->d_model, act_type(L->qt_gate)).bytes * (pt ? (size_t)n_tokens : P), sizeof(float) * P * L->d_ff,
+            ActLayout(L->d_model, act_type(L->qt_gate)).bytes * P, sizeof(float) * P * L->d_ff,
             ActLayout(L->d_ff, act_type(L->qt_down)).bytes * P, sizeof(float) * P * L->d_model};
 }
 // false inside a capture for which the scratch would have to grow

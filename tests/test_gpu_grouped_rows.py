@@ -214,3 +214,32 @@ def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, t
         graph.replay()
         torch.cuda.synchronize()
         assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
+
+
+def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
+    """An eager call that runs group-major leaves room for a smaller, token-major
+    call of the same layer inside a capture, which cannot allocate."""
+    from sabah.runtime import rt
+    E, K, D, F, tokens, small = 6, 3, 1024, 2304, 700, 5
+    rng = np.random.default_rng(77)
+    banks = [T(bank_bytes(rng, q, E, rows, k)) for q, rows, k in ((Q5_K, F, D), (Q5_K, F, D), (Q5_K, D, F))]
+    desc = rt.MoeLayerDesc()
+    desc.gate, desc.up, desc.down = (b.data_ptr() for b in banks)
+    desc.qt_gate = desc.qt_up = desc.qt_down = Q5_K
+    desc.d_model, desc.d_ff, desc.n_experts = D, F, E
+    x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(np.stack([rng.choice(E, K, replace=False) for _ in range(tokens)]).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    layer(hip_rt, "sabah_moe_layer", desc, x, ids, w)
+    want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x[:small], ids[:small], w[:small])
+    out = torch.empty_like(x[:small])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        hip_rt.check(hip_rt.lib().sabah_moe_layer(
+            ctypes.byref(desc), vp(x), vp(ids), vp(w), K, small, vp(out), None,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "captured layer")
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
