@@ -2268,8 +2268,9 @@ SABAH_API int sabah_moe_route(const float* d_logits, int n_tokens, int n_experts
     const dim3 grid((unsigned)n_tokens), block(kRouteThreads);
     hipStream_t st = pick_stream(stream);
     const int per = (n_experts + kRouteThreads - 1) / kRouteThreads;
-    if (per <= 1) hipLaunchKernelGGL(k_route<1>, grid, block, 0, st, a);
-    else if (per <= 2) hipLaunchKernelGGL(k_route<2>, grid, block, 0, st, a);
+    if (n_experts <= 64) hipLaunchKernelGGL(k_route_wave<1>, grid, dim3(64), 0, st, a);
+    else if (n_experts <= 128) hipLaunchKernelGGL(k_route_wave<2>, grid, dim3(64), 0, st, a);
+    else if (n_experts <= 512) hipLaunchKernelGGL(k_route_wave<8>, grid, dim3(64), 0, st, a);
     else if (per <= 4) hipLaunchKernelGGL(k_route<4>, grid, block, 0, st, a);
     else if (per <= 8) hipLaunchKernelGGL(k_route<8>, grid, block, 0, st, a);
     else hipLaunchKernelGGL(k_route<kRouteMaxPerThread>, grid, block, 0, st, a);

@@ -82,3 +82,21 @@ def test_routed_layer_from_device_logits(hip_rt, orc):
     assert np.array_equal(ids.cpu().numpy(), rid)
     want = orc.moe_layer(raws["gate"], raws["up"], raws["down"], (IQ3_S,) * 3, x, rid, rw)
     assert_parity(got, want, "routed layer")
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 8), (64, 64), (65, 6), (128, 64), (129, 8), (511, 10), (512, 64), (513, 10)])
+@pytest.mark.parametrize("norm_w", [True, False])
+def test_route_at_the_edges_of_the_one_wave_form(hip_rt, orc, E, k, norm_w):
+    """One wave routes a token up to 512 experts: expert counts about its
+    steps, the most picks, ties, minus infinity (a masked expert) and a wide
+    range of logits, against the oracle; weights as in the tests above."""
+    rng = np.random.default_rng(E + k)
+    logits = (rng.standard_normal((9, E)) * 1.5).astype(np.float32)
+    logits[1] = np.round(logits[1])
+    logits[2] *= 20
+    if E > 2 * k:
+        logits[3, ::2] = -np.inf
+    ids, w = route(hip_rt, logits, k, norm_w)
+    rid, rw = orc.moe_route(logits, k, norm_w, 1.0)
+    assert np.array_equal(ids, rid)
+    assert max_rel(w, rw) <= 2e-6
