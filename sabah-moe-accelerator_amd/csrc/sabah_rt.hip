@@ -977,6 +977,17 @@ static int grouped_mmid_form(int qt, bool packed, size_t ids_id_stride, size_t i
     return 0;
 }
 
+// kind < 0: not timed
+static void launch_group(int kind, const GroupArgs& a, hipStream_t st) {
+    const int lds = (int)sizeof(int) * (2 * a.n_experts + kGroupThreads);
+    auto go = [&](auto kernel) {
+        if (kind >= 0) launch_kernel(kind, kernel, dim3(1), dim3(kGroupThreads), lds, st, a);
+        else hipLaunchKernelGGL(kernel, dim3(1), dim3(kGroupThreads), lds, st, a);
+    };
+    if (a.n_tokens * a.k <= kGroupIdRegs * kGroupThreads) go(k_group_pairs<kGroupIdRegs>);
+    else go(k_group_pairs<2 * kGroupIdRegs>);
+}
+
 static int mmid_grouped(int form, int qt, const uint8_t* bank, size_t expert_stride, const float* d_x, int x_rows,
                         const int32_t* d_ids, int n_ids, int n_tokens, float* d_dst, size_t dst_id_stride,
                         size_t dst_token_stride, int rows, int k, int n_experts, hipStream_t st) {
@@ -992,8 +1003,7 @@ static int mmid_grouped(int form, int qt, const uint8_t* bank, size_t expert_str
     GroupArgs ga{d_ids, n_tokens, n_ids, E, off, pair_of, pos_of, g_err_dev, d_dst, dst_id_stride, dst_token_stride, rows};
     // the grouping and quantisation launches time as part of the call
     // (KK_MMID), so a call's kernel time covers all three of its launches
-    launch_kernel(KK_MMID, k_group_pairs, dim3(1), dim3(kGroupThreads), (int)sizeof(int) * (2 * E + kGroupThreads), st,
-                  ga);
+    launch_group(KK_MMID, ga, st);
     // the pairs' x rows, quantised in group order (pair p = t * n_ids + s reads x row p / x_div)
     const int x_div = x_rows == 1 ? n_ids : 1;
     const size_t xq_rows = P * (size_t)(k / 256);
@@ -1085,8 +1095,7 @@ static void launch_group_items(int kind, const RowsIndex& R, const int32_t* d_id
                                int pt, float* poison, size_t nb1, size_t nb2, int poison_rows, hipStream_t st) {
     GroupArgs ga{d_ids, n_tokens, k, n_experts, R.off, R.pair_of, R.pos_of, g_err_dev, poison, nb1, nb2, poison_rows,
                  R.items, R.n_items, 16 * pt};
-    launch_kernel(kind, k_group_pairs, dim3(1), dim3(kGroupThreads), (int)sizeof(int) * (2 * n_experts + kGroupThreads), st,
-                  ga);
+    launch_group(kind, ga, st);
 }
 // rows [n][k] -> q8 rows of the weight type's activation format, in MFMA operand order
 static void launch_quant_mfma(int kind, const float* x, size_t n, int k, int qt, uint8_t* out, int stride,
@@ -2173,7 +2182,7 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
         launch_rows<kRowsOut>(L->qt_down, KK_GDOWN, pt, items, ga, st);
     } else {
         GroupArgs ga{d_ids, n_tokens, n_used, E, off, pair_of, pos_of, g_err_dev, nullptr, 0, 0, 0, nullptr, nullptr, 0};
-        hipLaunchKernelGGL(k_group_pairs, dim3(1), dim3(kGroupThreads), sizeof(int) * (2 * E + kGroupThreads), st, ga);
+        launch_group(-1, ga, st);
         // the pairs' x rows in group order (pair p is token p / n_used)
         const size_t xq_rows = P * (size_t)(D / 256);
         hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((xq_rows + 15) / 16)), dim3(kThreads), 0, st, d_x, (int)P, D,
