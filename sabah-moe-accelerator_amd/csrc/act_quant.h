@@ -224,7 +224,8 @@ __device__ inline void load16(const float* row, int e, int k, bool vec, Act16& a
 }
 
 // An activation batch: n_rows rows of k floats, row_stride floats apart,
-// quantised into ActLayout blocks act_stride bytes apart.  Chunk-row q (row
+// quantised into ActLayout blocks act_stride bytes apart (act_quantize: in LDS,
+// so every offset is small).  Chunk-row q (row
 // q / nch, chunk q % nch) belongs to row-slot q % nslots (a row-slot is one
 // 16-lane DPP row of the workgroup) in round q / nslots.
 struct ActBatch {
@@ -265,34 +266,36 @@ __device__ inline void act_prefetch(const ActBatch& B, ActRegs<ROUNDS>& R, int w
     }
 }
 
-__device__ inline void quant_chunk(const ActBatch& B, const Act16& a_in, int q, int mfma_order = 0) {
-    const int nch = (B.k + 255) / 256;
-    const int r = div_small(q, __builtin_amdgcn_rcpf((float)nch)), c = q - r * nch;
+// chunk c of a row, held as Act16, into the row's ActLayout block
+__device__ inline void quant_chunk(const ActBatch& B, const Act16& a_in, int c, uint8_t* row, int mfma_order = 0) {
     const ActLayout L(B.k, B.at);
     const bool in = c * 256 + 16 * (int)(threadIdx.x & 15u) < B.k;
     Act16 a;
 #pragma unroll
     for (int j = 0; j < 16; ++j) a.v[j] = in ? a_in.v[j] : 0.0f;
-    if (B.at == QT_Q8_K) row16_quant_q8K(a, c, B.act + r * B.act_stride, L, mfma_order);
-    else row16_quant_q8_0(a, c, B.act + r * B.act_stride, L, B.at == QT_Q8_1, mfma_order);
+    if (B.at == QT_Q8_K) row16_quant_q8K(a, c, row, L, mfma_order);
+    else row16_quant_q8_0(a, c, row, L, B.at == QT_Q8_1, mfma_order);
 }
 
 template <int ROUNDS, int NT>
 __device__ inline void act_quantize(const ActBatch& B, const ActRegs<ROUNDS>& R, int w0 = 0) {
     const int slot = ((int)threadIdx.x - w0) >> 4, nslots = (NT - w0) >> 4, l = threadIdx.x & 15;
     const int nch = (B.k + 255) / 256, nq = B.n_rows * nch;
+    const float rcp_nch = __builtin_amdgcn_rcpf((float)nch);
 #pragma unroll
     for (int i = 0; i < ROUNDS; ++i) {
         const int q = slot + nslots * i;
-        if (q < nq) quant_chunk(B, R.a[i], q);
+        if (q < nq) {
+            const int r = div_small(q, rcp_nch);
+            quant_chunk(B, R.a[i], q - r * nch, B.act + r * B.act_stride);
+        }
     }
     const bool vec = act_vec(B);
-    const float rcp_nch = __builtin_amdgcn_rcpf((float)nch);
     for (int q = slot + nslots * ROUNDS; q < nq; q += nslots) {
         const int r = div_small(q, rcp_nch), c = q - r * nch;
         Act16 a;
         load16(B.x + (size_t)r * B.row_stride, c * 256 + 16 * l, B.k, vec, a);
-        quant_chunk(B, a, q);
+        quant_chunk(B, a, c, B.act + r * B.act_stride);
     }
 }
 

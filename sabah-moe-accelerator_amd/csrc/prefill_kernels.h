@@ -182,13 +182,13 @@ __global__ __launch_bounds__(kThreads) void k_quant_rows(const float* __restrict
     const int nch = (k + 255) / 256;
     const int q = blockIdx.x * (kThreads / 16) + (int)(threadIdx.x >> 4);
     if (q >= n_rows * nch) return;                       // whole 16-lane rows leave together
-    const int r = q / nch, c = q - r * nch;
-    if (count && r >= *count) return;
-    const int src = gather ? gather[r] / gdiv : r;
+    const ChunkPlace P = chunk_place(q, nch, out_stride);
+    if (count && P.row >= *count) return;
+    const int src = gather ? gather[P.row] / gdiv : P.row;
     const ActBatch B{x, (size_t)k, n_rows, k, at, out, out_stride};
     Act16 v;
-    load16(x + (size_t)src * k, c * 256 + 16 * (int)(threadIdx.x & 15u), k, act_vec(B), v);
-    quant_chunk(B, v, q, mfma_order);
+    load16(x + (size_t)src * k, P.chunk * 256 + 16 * (int)(threadIdx.x & 15u), k, act_vec(B), v);
+    quant_chunk(B, v, P.chunk, out + P.offset, mfma_order);
 }
 
 // ---------------------------------------------------------------------------

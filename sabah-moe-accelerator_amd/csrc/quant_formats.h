@@ -143,4 +143,17 @@ struct ActLayout {
     }
 };
 
+// Chunk-row q of a batch of rows of nch chunks, `stride` bytes apart in memory:
+// its row, its chunk of that row and the row's byte offset.  A large call's
+// rows are millions of chunks and gigabytes in all: an exact division and a
+// 64-bit product.
+struct ChunkPlace {
+    int row, chunk;
+    size_t offset;
+};
+__host__ __device__ inline ChunkPlace chunk_place(int q, int nch, int stride) {
+    const int r = q / nch;
+    return {r, q - r * nch, (size_t)r * (size_t)stride};
+}
+
 }  // namespace sabah

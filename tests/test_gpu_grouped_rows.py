@@ -243,3 +243,40 @@ def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
         graph.replay()
         torch.cuda.synchronize()
         assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
+
+
+# q8 rows past 2 GiB and past 2^21 chunks in all: in the general form with one x row
+# per slot (450,000 rows of 4,864 bytes) and in the fixed-shape form (900,000 of 2,464)
+@pytest.mark.parametrize("qt,k,tokens,K,slot_rows", [(Q8_0, 4096, 45000, 10, True), (Q4_K, 2048, 45000, 20, False)])
+def test_quantised_rows_past_2_gib(hip_rt, grouping, qt, k, tokens, K, slot_rows):
+    E, rows = 16, 64
+    rng = np.random.default_rng(k)
+    bank = T(bank_bytes(rng, qt, E, rows, k))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    g = torch.Generator(device=DEV).manual_seed(k)
+    x = torch.randn((tokens, K if slot_rows else 1, k), device=DEV, generator=g)
+    grouping(NEVER)
+    tok = mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped=False)
+    grouping(AUTO)
+    got = mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped=True)
+    assert_bits_equal(got, tok, "qt=%d" % qt)
+
+
+def test_a_layers_quantised_h_rows_past_2_gib(hip_rt):
+    """One run of 65,000 pairs at d_ff 28,672: 2.2 GB of q8 rows of h."""
+    from sabah.runtime import rt
+    E, K, D, F, tokens = 4, 1, 64, 28672, 65000
+    rng = np.random.default_rng(28)
+    banks = [T(bank_bytes(rng, Q8_0, E, rows, k)) for rows, k in ((F, D), (F, D), (D, F))]
+    desc = rt.MoeLayerDesc()
+    desc.gate, desc.up, desc.down = (b.data_ptr() for b in banks)
+    desc.qt_gate = desc.qt_up = desc.qt_down = Q8_0
+    desc.d_model, desc.d_ff, desc.n_experts = D, F, E
+    x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    got = layer(hip_rt, "sabah_moe_layer", desc, x, ids, w)
+    for t in (0, 20000, 40000, tokens - 40):
+        s = slice(t, t + 40)                      # as many tokens as the token-major call's static scratch holds
+        want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x[s].contiguous(), ids[s].contiguous(), w[s].contiguous())
+        assert_bits_equal(got[s], want, "tokens from %d" % t)
