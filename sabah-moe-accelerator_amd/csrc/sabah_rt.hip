@@ -189,16 +189,26 @@ bool stream_capturing(hipStream_t st) {
     return cs != hipStreamCaptureStatusNone;
 }
 
-void* grow_scratch(Scratch& s, size_t bytes, hipStream_t stream) {
-    if (s.bytes >= bytes) return s.p;
+// tests only (sabah_rt_set_scratch_refusal): the device refuses all optional scratch
+std::atomic<bool> g_scratch_refusal{false};
+
+// optional: the caller has another form that needs none
+void* grow_scratch(Scratch& s, size_t bytes, hipStream_t stream, bool optional = false) {
+    const bool refuse = optional && g_scratch_refusal.load();
+    if (s.bytes >= bytes && !refuse) return s.p;
     if (stream_capturing(stream)) {
         fail("library scratch must grow to %zu bytes (from %zu) during a stream capture, which cannot "
              "allocate: make the same call once before the capture", bytes, s.bytes);
         return nullptr;
     }
     size_t want = std::max(bytes, std::max(2 * s.bytes, (size_t)1 << 20));
+    if (refuse) want = (size_t)1 << 60;                     // more than any device has
     void* p = nullptr;
-    if (!ck(hipMalloc(&p, want), "scratch allocation")) return nullptr;
+    if (!ck(hipMalloc(&p, want), "scratch allocation")) {
+        // the runtime keeps the failure as the thread's last error, which the next launch's check would read
+        (void)hipGetLastError();
+        return nullptr;
+    }
     std::lock_guard<std::mutex> lk(g_retired_mu);
     if (s.p) g_retired.push_back(s.p);
     s.p = p;
@@ -661,6 +671,14 @@ SABAH_API int sabah_rt_set_layer_fusion(int mode) {
 SABAH_API int sabah_rt_set_mmid_rounds(int mode) {
     if (mode < 0 || mode > 1) return fail("MUL_MAT_ID rounds mode %d outside {0 off, 1 on}", mode);
     g_mmid_rounds.store(mode);
+    return 0;
+}
+
+// Tests of the calls that do without their optional scratch: on, every
+// allocation of scratch that a call has another form without (the general grouped
+// form's) asks the device for more than it has and is refused.
+SABAH_API int sabah_rt_set_scratch_refusal(int on) {
+    g_scratch_refusal.store(on != 0);
     return 0;
 }
 
@@ -1193,7 +1211,7 @@ static RowsWorkspace* rows_workspace(size_t index_bytes, size_t xq_bytes, hipStr
         w = &g_rows_ws.back();
         w->st = st;
     }
-    return grow_scratch(w->index, index_bytes, st) && grow_scratch(w->xq, xq_bytes, st) ? w : nullptr;
+    return grow_scratch(w->index, index_bytes, st, true) && grow_scratch(w->xq, xq_bytes, st, true) ? w : nullptr;
 }
 // 0 done, -1 error, 1 not here: the call takes the token-major kernel.  These
 // calls never take the grouped form inside a capture (a replay would use the stream's
@@ -2119,11 +2137,12 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
     const int xq_stride = (int)ActLayout(D, act_type(L->qt_gate)).bytes;
     const int hq_stride = (int)ActLayout(F, act_type(L->qt_down)).bytes;
     const GroupedBufs B = grouped_bufs(L, n_used, n_tokens, pt);
-    void* index = grow_scratch(g_scratch_goff, B.index, st);
-    uint8_t* xq = static_cast<uint8_t*>(grow_scratch(g_scratch_gxq, B.xq, st));
-    float* h = static_cast<float*>(grow_scratch(g_scratch_gh, B.h, st));
-    uint8_t* hq = static_cast<uint8_t*>(grow_scratch(g_scratch_ghq, B.hq, st));
-    float* y = static_cast<float*>(grow_scratch(g_scratch_gy, B.y, st));
+    const bool optional = pt != 0;
+    void* index = grow_scratch(g_scratch_goff, B.index, st, optional);
+    uint8_t* xq = static_cast<uint8_t*>(grow_scratch(g_scratch_gxq, B.xq, st, optional));
+    float* h = static_cast<float*>(grow_scratch(g_scratch_gh, B.h, st, optional));
+    uint8_t* hq = static_cast<uint8_t*>(grow_scratch(g_scratch_ghq, B.hq, st, optional));
+    float* y = static_cast<float*>(grow_scratch(g_scratch_gy, B.y, st, optional));
     if (!index || !xq || !h || !hq || !y) return pt ? 1 : -1;
     const RowsIndex R = rows_index(index, P, E, pt ? pt : 2);
     int *const off = R.off, *const pair_of = R.pair_of, *const pos_of = R.pos_of;

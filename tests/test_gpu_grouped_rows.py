@@ -280,3 +280,34 @@ def test_a_layers_quantised_h_rows_past_2_gib(hip_rt):
         s = slice(t, t + 40)                      # as many tokens as the token-major call's static scratch holds
         want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x[s].contiguous(), ids[s].contiguous(), w[s].contiguous())
         assert_bits_equal(got[s], want, "tokens from %d" % t)
+
+
+def test_calls_whose_optional_scratch_is_refused_run_token_major(hip_rt, grouping):
+    """A device with no room for the grouped form's scratch: the call and the
+    layer take the kernels that need none, and no error is left for either."""
+    from sabah.runtime import rt
+    lib = hip_rt.lib()
+    E, K, D, F, tokens = 6, 2, 512, 256, 301
+    rng = np.random.default_rng(91)
+    banks = [T(bank_bytes(rng, Q5_K, E, rows, k)) for rows, k in ((F, D), (F, D), (D, F))]
+    desc = rt.MoeLayerDesc()
+    desc.gate, desc.up, desc.down = (b.data_ptr() for b in banks)
+    desc.qt_gate = desc.qt_up = desc.qt_down = Q5_K
+    desc.d_model, desc.d_ff, desc.n_experts = D, F, E
+    x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    x3 = x.view(tokens, 1, D)
+    want = mmid(hip_rt, banks[0], Q5_K, F, D, E, x3, ids, grouped=True)
+    want_layer = layer(hip_rt, "sabah_moe_layer", desc, x, ids, w)
+    hip_rt.check(lib.sabah_rt_set_scratch_refusal(1), "refusal on")
+    hip_rt.check(lib.sabah_rt_set_kernel_timing(1), "timing on")
+    try:
+        assert_bits_equal(mmid(hip_rt, banks[0], Q5_K, F, D, E, x3, ids, grouped=False), want, "MUL_MAT_ID")
+        grouped_launches(hip_rt)
+        assert_bits_equal(layer(hip_rt, "sabah_moe_layer", desc, x, ids, w), want_layer, "layer")
+        assert grouped_launches(hip_rt) == 0
+    finally:
+        lib.sabah_rt_set_kernel_timing(0)
+        lib.sabah_rt_set_scratch_refusal(0)
+    assert_bits_equal(mmid(hip_rt, banks[0], Q5_K, F, D, E, x3, ids, grouped=True), want, "grouped again")
