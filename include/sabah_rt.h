@@ -291,7 +291,9 @@ int sabah_moe_route(const float *d_logits, int n_tokens, int n_experts, int n_us
  * == 0, use library scratch (pair lists, q8 rows) shared by every stream when
  * grouped: such calls that may overlap on different streams need mode 1 (the
  * token-major kernel uses no scratch).  All other grouped calls use a
- * workspace of their stream, and inside a stream capture run token-major.
+ * workspace of their stream (eight in all; a further stream takes over the least
+ * recently used one, after its last call), and inside a stream capture and on the
+ * per-thread default stream run token-major.
  * Returns -1 for another mode. */
 int sabah_rt_set_mmid_grouping(int mode);
 

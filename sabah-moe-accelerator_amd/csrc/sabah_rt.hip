@@ -100,13 +100,19 @@ Scratch g_scratch_sxq, g_scratch_shq, g_scratch_sgl;
 Scratch g_scratch_goff, g_scratch_gpair, g_scratch_gxq, g_scratch_gh, g_scratch_ghq, g_scratch_gy;
 // MUL_MAT_ID through k_grouped_rows: one workspace per stream (calls on
 // different streams may overlap), at most kMaxRowsStreams of them, kept until
-// sabah_rt_shutdown; g_rows_mu is held while a call that uses one is enqueued
+// sabah_rt_shutdown; a further stream takes over the least recently used one.
+// Every call waits for the workspace's last one (done), which may have run on
+// another stream, or on a destroyed one whose handle this stream got.
+// g_rows_mu is held while a call that uses one is enqueued.
 struct RowsWorkspace {
     hipStream_t st = nullptr;
     Scratch index, xq;
+    hipEvent_t done = nullptr;         // recorded after the last call
+    unsigned long long last = 0;       // g_rows_clock at the last call
 };
 constexpr size_t kMaxRowsStreams = 8;
 std::vector<RowsWorkspace> g_rows_ws;
+unsigned long long g_rows_clock = 0;
 std::mutex g_rows_mu;
 uint16_t* g_nearest_dev = nullptr;   // IQ3_S encoder table, uploaded on first use
 
@@ -150,6 +156,18 @@ void launch_kernel(int kind, K kernel, dim3 grid, dim3 block, int lds, hipStream
         }
     }
     hipLaunchKernelGGL(kernel, grid, block, lds, st, args...);
+}
+
+// The same, and `done` (or null) is recorded as the kernel ends: the dispatch's own
+// stop event where the launch carries no timing events
+template <typename K, typename... A>
+void launch_kernel_done(hipEvent_t done, int kind, K kernel, dim3 grid, dim3 block, int lds, hipStream_t st, A... args) {
+    if (done && !(g_timing.load() && !g_launch_plain)) {
+        hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)lds, st, nullptr, done, 0u, args...);
+        return;
+    }
+    launch_kernel(kind, kernel, grid, block, lds, st, args...);
+    if (done) (void)hipEventRecord(done, st);               // an error is the launch check's to report
 }
 
 int fail(const char* fmt, ...) {
@@ -605,9 +623,11 @@ SABAH_API int sabah_rt_shutdown(void) {
     }
     {
         std::lock_guard<std::mutex> lk(g_rows_mu);
-        for (RowsWorkspace& w : g_rows_ws)
+        for (RowsWorkspace& w : g_rows_ws) {
             for (Scratch* s : {&w.index, &w.xq})
                 if (s->p) (void)hipFree(s->p);
+            (void)hipEventDestroy(w.done);
+        }
         g_rows_ws.clear();
     }
     for (void* p : g_retired) (void)hipFree(p);
@@ -1131,17 +1151,18 @@ static int rows_groups(int qt, int pt, int rows, size_t items) {
     return qt != QT_Q8_0 && pt == 2 && tiles * 2 * kRowsTile <= rows + rows / 8 && (size_t)tiles * items >= 1024 ? 2 : 1;
 }
 template <int G, int MODE>
-static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
+static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st,
+                          hipEvent_t done) {
     const int tile = MODE == kRowsSwiglu ? kRowsTile : G * kRowsTile;
     const dim3 grid((unsigned)((a.rows + tile - 1) / tile), (unsigned)items);
-#define SB_ROWS(QT)                                                                                       \
-    case QT:                                                                                               \
-        if constexpr (G == 1 || (MODE == kRowsSwiglu && QT != QT_Q8_0))                                    \
-            if (pt == 4) {                                                                                 \
-                launch_kernel(kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a);       \
-                break;                                                                                     \
-            }                                                                                              \
-        launch_kernel(kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);               \
+#define SB_ROWS(QT)                                                                                           \
+    case QT:                                                                                                   \
+        if constexpr (G == 1 || (MODE == kRowsSwiglu && QT != QT_Q8_0))                                        \
+            if (pt == 4) {                                                                                     \
+                launch_kernel_done(done, kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a);    \
+                break;                                                                                         \
+            }                                                                                                  \
+        launch_kernel_done(done, kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);        \
         break;
     switch (qt) {
     SB_ROWS(QT_Q8_0)
@@ -1155,11 +1176,13 @@ static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedR
     }
 #undef SB_ROWS
 }
+// done: recorded as the kernel ends (or null)
 template <int MODE>
-static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st) {
-    if constexpr (MODE == kRowsSwiglu) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st);
-    else if (rows_groups(qt, pt, a.rows, items) == 2) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st);
-    else launch_rows_g<1, MODE>(qt, kind, pt, items, a, st);
+static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st,
+                        hipEvent_t done = nullptr) {
+    if constexpr (MODE == kRowsSwiglu) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st, done);
+    else if (rows_groups(qt, pt, a.rows, items) == 2) launch_rows_g<2, MODE>(qt, kind, pt, items, a, st, done);
+    else launch_rows_g<1, MODE>(qt, kind, pt, items, a, st, done);
 }
 
 // Where the general grouped form is the faster one: from base pairs (for
@@ -1199,17 +1222,31 @@ static bool mmid_rows_ok(int qt, bool packed, const uint8_t* bank, size_t expert
            x_token_stride == 4 * (size_t)k * x_rows && rows_bank_ok(bank, expert_stride) &&
            rows_shape_ok(qt, (size_t)n_tokens * n_ids, n_experts, rows, k);
 }
-// the stream's workspace, grown to the call's sizes; null: no more streams or
-// no memory (the token-major kernel needs neither)
+// the stream's workspace, grown to the call's sizes and free for it in stream order;
+// null: no memory (the token-major kernel needs none)
 static RowsWorkspace* rows_workspace(size_t index_bytes, size_t xq_bytes, hipStream_t st) {
     RowsWorkspace* w = nullptr;
     for (RowsWorkspace& v : g_rows_ws)
         if (v.st == st) w = &v;
-    if (!w) {
-        if (g_rows_ws.size() >= kMaxRowsStreams) return nullptr;
-        g_rows_ws.push_back({});
+    if (!w && g_rows_ws.size() < kMaxRowsStreams) {
+        // The event orders kernels of one device, which needs no system fence, and is
+        // the last dispatch's own stop event.  A Q8_0 down node (301 tokens), us per call: 30.1 with no event,
+        // 30.2 - 30.8 so, 32.1 with the fence, 31.4 recorded by itself, 32.9 by itself with the fence.
+        RowsWorkspace v;
+        if (hipEventCreateWithFlags(&v.done, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        g_rows_ws.push_back(v);
         w = &g_rows_ws.back();
-        w->st = st;
+    }
+    if (!w)
+        w = &*std::min_element(g_rows_ws.begin(), g_rows_ws.end(),
+                               [](const RowsWorkspace& a, const RowsWorkspace& b) { return a.last < b.last; });
+    w->st = st;
+    if (w->last && hipStreamWaitEvent(st, w->done, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
     }
     return grow_scratch(w->index, index_bytes, st, true) && grow_scratch(w->xq, xq_bytes, st, true) ? w : nullptr;
 }
@@ -1245,7 +1282,8 @@ static int mmid_rows(int qt, const uint8_t* bank, size_t expert_stride, const fl
     a.dst_nb1 = dst_id_stride;
     a.dst_nb2 = dst_token_stride;
     a.n_ids = n_ids;
-    launch_rows<kRowsMmid>(qt, KK_MMID, pt, rows_item_bound(P, n_experts, pt), a, st);
+    launch_rows<kRowsMmid>(qt, KK_MMID, pt, rows_item_bound(P, n_experts, pt), a, st, w->done);
+    w->last = ++g_rows_clock;
     return ck(hipGetLastError(), "grouped MUL_MAT_ID launch") ? 0 : -1;
 }
 

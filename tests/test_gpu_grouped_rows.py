@@ -155,6 +155,58 @@ def test_calls_on_two_streams_and_under_capture(hip_rt, grouping):
     assert hip_rt.snapshot()["grouped_calls"] == before + 20
 
 
+def hip_runtime():
+    """The HIP runtime this process runs on."""
+    with open("/proc/self/maps") as f:
+        return ctypes.CDLL(next(l.split()[-1] for l in f if "libamdhip64" in l))
+
+
+@pytest.mark.parametrize("kind", ["twelve", "created and destroyed", "per thread"])
+def test_more_streams_than_workspaces(hip_rt, grouping, kind):
+    """Eight workspaces serve any number of streams: a further stream takes over
+    the least recently used one, in order after its last call, and a
+    destroyed stream holds none.  The per-thread default stream (one handle for every
+    thread) is served token-major."""
+    E, K, rows, k = 7, 2, 960, 768
+    rng = np.random.default_rng(61)
+    bank = T(bank_bytes(rng, IQ3_XXS, E, rows, k))
+    lib, rb = hip_rt.lib(), hip_rt.row_bytes(IQ3_XXS, k)
+    tokens = [200, 130, 333, 150]
+    xs = [T(rng.standard_normal((t, 1, k)).astype(np.float32)) for t in tokens]
+    ids = [T(rng.integers(0, E, (t, K)).astype(np.int32)) for t in tokens]
+    grouping(NEVER)
+    want = [mmid(hip_rt, bank, IQ3_XXS, rows, k, E, x, i, grouped=False) for x, i in zip(xs, ids)]
+    grouping(AUTO)
+
+    def call(i, out, handle):
+        hip_rt.check(lib.sabah_rt_mul_mat_id_v2(
+            vp(bank), ctypes.c_size_t(rows * rb), ctypes.c_size_t(rb), vp(xs[i]), ctypes.c_size_t(k * 4), 1,
+            ctypes.c_size_t(k * 4), vp(ids[i]), ctypes.c_size_t(4), ctypes.c_size_t(K * 4), K, tokens[i], vp(out),
+            ctypes.c_size_t(rows * 4), ctypes.c_size_t(K * rows * 4), rows, k, E, IQ3_XXS,
+            ctypes.c_void_p(handle), None), "v2")
+
+    n = 36
+    outs = [torch.zeros(tokens[j % 4], K, rows, device=DEV) for j in range(n)]
+    streams = [torch.cuda.Stream() for _ in range(12)]
+    torch.cuda.synchronize()
+    before = hip_rt.snapshot()["grouped_calls"]
+    hip = hip_runtime()
+    for j in range(n):                                  # back to back: nothing waits on the host
+        if kind == "twelve":
+            call(j % 4, outs[j], streams[j % 12].cuda_stream)
+        elif kind == "per thread":
+            call(j % 4, outs[j], 2)                     # hipStreamPerThread
+        else:
+            h = ctypes.c_void_p()
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(h), 1) == 0
+            call(j % 4, outs[j], h.value)
+            assert hip.hipStreamDestroy(h) == 0
+    torch.cuda.synchronize()
+    assert hip_rt.snapshot()["grouped_calls"] == before + (0 if kind == "per thread" else n)
+    for j in range(n):
+        assert_bits_equal(outs[j].cpu().numpy(), want[j % 4], "call %d" % j)
+
+
 def grouped_launches(hip_rt):
     """Group-major gate/up launches (kernel kind 4) since the last reading, with timing on."""
     ms, n = ctypes.c_double(), ctypes.c_ulonglong()
