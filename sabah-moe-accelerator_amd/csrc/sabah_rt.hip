@@ -207,6 +207,15 @@ bool stream_capturing(hipStream_t st) {
     return cs != hipStreamCaptureStatusNone;
 }
 
+// While one lives, its thread may allocate although another stream is being
+// captured in the global or the thread's mode; without it the allocation fails and ends
+// that capture.  The call's own stream is not capturing (grow_scratch checks).
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // tests only (sabah_rt_set_scratch_refusal): the device refuses all optional scratch
 std::atomic<bool> g_scratch_refusal{false};
 
@@ -222,6 +231,7 @@ void* grow_scratch(Scratch& s, size_t bytes, hipStream_t stream, bool optional =
     size_t want = std::max(bytes, std::max(2 * s.bytes, (size_t)1 << 20));
     if (refuse) want = (size_t)1 << 60;                     // more than any device has
     void* p = nullptr;
+    const RelaxedCapture relaxed;
     if (!ck(hipMalloc(&p, want), "scratch allocation")) {
         // the runtime keeps the failure as the thread's last error, which the next launch's check would read
         (void)hipGetLastError();
@@ -1232,6 +1242,7 @@ static RowsWorkspace* rows_workspace(size_t index_bytes, size_t xq_bytes, hipStr
         // The event orders kernels of one device, which needs no system fence, and is
         // the last dispatch's own stop event.  A Q8_0 down node (301 tokens), us per call: 30.1 with no event,
         // 30.2 - 30.8 so, 32.1 with the fence, 31.4 recorded by itself, 32.9 by itself with the fence.
+        const RelaxedCapture relaxed;
         RowsWorkspace v;
         if (hipEventCreateWithFlags(&v.done, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
             (void)hipGetLastError();

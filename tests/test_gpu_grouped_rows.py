@@ -207,6 +207,42 @@ def test_more_streams_than_workspaces(hip_rt, grouping, kind):
         assert_bits_equal(outs[j].cpu().numpy(), want[j % 4], "call %d" % j)
 
 
+def test_a_call_that_allocates_beside_another_streams_capture(hip_rt, grouping):
+    """A first call on its stream, whose workspace has to be allocated, while another
+    stream is being captured: both go through."""
+    E, K, rows, k, tokens = 7, 2, 960, 768, 20000      # larger than the other tests' workspaces
+    rng = np.random.default_rng(62)
+    bank = T(bank_bytes(rng, IQ3_XXS, E, rows, k))
+    lib, rb = hip_rt.lib(), hip_rt.row_bytes(IQ3_XXS, k)
+    x = T(rng.standard_normal((tokens, 1, k)).astype(np.float32))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    grouping(NEVER)
+    want = mmid(hip_rt, bank, IQ3_XXS, rows, k, E, x, ids, grouped=False)
+    grouping(AUTO)
+    out = torch.zeros(tokens, K, rows, device=DEV)
+    other, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    a, b = torch.ones(1000, device=DEV), torch.zeros(1000, device=DEV)
+    torch.cuda.synchronize()
+    before = hip_rt.snapshot()
+    with torch.cuda.graph(graph):
+        torch.add(a, 1.0, out=b)
+        hip_rt.check(lib.sabah_rt_mul_mat_id_v2(
+            vp(bank), ctypes.c_size_t(rows * rb), ctypes.c_size_t(rb), vp(x), ctypes.c_size_t(k * 4), 1,
+            ctypes.c_size_t(k * 4), vp(ids), ctypes.c_size_t(4), ctypes.c_size_t(K * 4), K, tokens, vp(out),
+            ctypes.c_size_t(rows * 4), ctypes.c_size_t(K * rows * 4), rows, k, E, IQ3_XXS,
+            ctypes.c_void_p(other.cuda_stream), None), "v2")
+    torch.cuda.synchronize()
+    after = hip_rt.snapshot()
+    assert after["grouped_calls"] == before["grouped_calls"] + 1
+    assert after["scratch_bytes"] > before["scratch_bytes"]
+    assert_bits_equal(out.cpu().numpy(), want, "the eager call")
+    for _ in range(3):
+        b.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (b == 2.0).all()
+
+
 def grouped_launches(hip_rt):
     """Group-major gate/up launches (kernel kind 4) since the last reading, with timing on."""
     ms, n = ctypes.c_double(), ctypes.c_ulonglong()
