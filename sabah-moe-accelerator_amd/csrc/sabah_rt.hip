@@ -1745,8 +1745,7 @@ static size_t layer_scratch_bytes(const sabah_moe_layer_desc* L, int n_used, int
     if (const size_t hq = layer_hq_bytes(L, n_used, n_tokens)) take(hq);
     return used;
 }
-static int layer_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, Workspace& ws, hipStream_t st,
-                      LayerBufs& b) {
+static int shared_bufs(const sabah_moe_layer_desc* L, int n_tokens, Workspace& ws, hipStream_t st, LayerBufs& b) {
     if (L->shared_gate) {
         b.hs = static_cast<float*>(ws.get(g_scratch_hs, sizeof(float) * (size_t)n_tokens * L->d_ff_shared, st));
         b.ys = static_cast<float*>(ws.get(g_scratch_ys, sizeof(float) * (size_t)n_tokens * L->d_model, st));
@@ -1760,6 +1759,11 @@ static int layer_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, W
         b.sgl = static_cast<float*>(ws.get(g_scratch_sgl, sizeof(float) * (size_t)n_tokens, st));
         if (!b.sxq || !b.shq || !b.sgl) return -1;
     }
+    return 0;
+}
+static int layer_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, Workspace& ws, hipStream_t st,
+                      LayerBufs& b) {
+    if (shared_bufs(L, n_tokens, ws, st, b)) return -1;
     b.h = static_cast<float*>(ws.get(g_scratch_h, sizeof(float) * (size_t)n_tokens * n_used * L->d_ff, st));
     if (!b.h) return -1;
     if (const size_t hq = layer_hq_bytes(L, n_used, n_tokens)) {
@@ -2004,14 +2008,25 @@ static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_token
 }
 static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                           int n_used, int n_tokens, float* d_out, const float* d_resid, int pt, hipStream_t st);
-static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st);
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, hipStream_t st);
+// the largest batch below n_tokens that is not one of `takes` (which is true from
+// some size on, and of n_tokens, and never of one token)
+template <typename F>
+static int largest_other(int n_tokens, F takes) {
+    int lo = 1, hi = n_tokens;
+    while (hi - lo > 1) {
+        const int mid = lo + (hi - lo) / 2;
+        (takes(mid) ? hi : lo) = mid;
+    }
+    return lo;
+}
 // 0 done, -1 error, 1 not here (the token-major kernels)
 static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                           int n_used, int n_tokens, float* d_out, const float* d_resid, hipStream_t st) {
     if (!rows_layer_ok(L, n_used, n_tokens)) return 1;
     const int run = rows_run(n_used, n_tokens);
     const int pt = rows_tiles((size_t)run * n_used, L->n_experts, L->d_ff, L->qt_gate == QT_Q8_0);
-    if (!grouped_layer_ready(L, n_used, run, pt, st)) return 1;
+    if (!grouped_layer_ready(L, n_used, run, st)) return 1;
     for (int t = 0; t < n_tokens; t += run) {
         const size_t td = (size_t)t * L->d_model, tk = (size_t)t * n_used;
         const int rc = moe_grouped_on(L, d_x + td, d_ids + tk, d_w + tk, n_used, std::min(run, n_tokens - t), d_out + td,
@@ -2158,13 +2173,15 @@ static bool grouped_shape_ok(const sabah_moe_layer_desc* L) {
 // Scratch of a group-major layer.  pt = 0: the fixed-shape kernels' (the
 // pairs' x rows quantised in group order); pt = 2, 4: k_grouped_rows with items of pt
 // 16-pair tiles (one q8 row per token; xq is sized for the pairs all the same,
-// so a smaller call that takes the other kernels finds its room in a capture).
+// so a smaller call that takes the other kernels finds its room in a capture).  The index
+// is sized for two-tile items, the more of the two, so that no smaller batch needs more than
+// a larger one.
 struct GroupedBufs {
     size_t index, xq, h, hq, y;
 };
-static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt) {
+static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
     const size_t P = (size_t)n_tokens * n_used;
-    return {rows_index_bytes(P, L->n_experts, pt ? pt : 2),
+    return {rows_index_bytes(P, L->n_experts, 2),
             ActLayout(L->d_model, act_type(L->qt_gate)).bytes * P, sizeof(float) * P * L->d_ff,
             ActLayout(L->d_ff, act_type(L->qt_down)).bytes * P, sizeof(float) * P * L->d_model};
 }
@@ -2174,8 +2191,14 @@ static bool grouped_scratch_ready(const GroupedBufs& B, hipStream_t st) {
             g_scratch_ghq.bytes >= B.hq && g_scratch_gy.bytes >= B.y) || !stream_capturing(st);
 }
 
-static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st) {
-    return grouped_scratch_ready(grouped_bufs(L, n_used, n_tokens, pt), st);
+static bool grouped_scratch(const GroupedBufs& B, hipStream_t st, bool optional = false) {
+    return grow_scratch(g_scratch_goff, B.index, st, optional) && grow_scratch(g_scratch_gxq, B.xq, st, optional) &&
+           grow_scratch(g_scratch_gh, B.h, st, optional) && grow_scratch(g_scratch_ghq, B.hq, st, optional) &&
+           grow_scratch(g_scratch_gy, B.y, st, optional);
+}
+
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, hipStream_t st) {
+    return grouped_scratch_ready(grouped_bufs(L, n_used, n_tokens), st);
 }
 
 // 0 done, -1 error, 1 (pt > 0 only) nothing launched: no memory for the scratch
@@ -2185,38 +2208,23 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
     const size_t P = (size_t)n_tokens * n_used;
     const int xq_stride = (int)ActLayout(D, act_type(L->qt_gate)).bytes;
     const int hq_stride = (int)ActLayout(F, act_type(L->qt_down)).bytes;
-    const GroupedBufs B = grouped_bufs(L, n_used, n_tokens, pt);
-    const bool optional = pt != 0;
-    void* index = grow_scratch(g_scratch_goff, B.index, st, optional);
-    uint8_t* xq = static_cast<uint8_t*>(grow_scratch(g_scratch_gxq, B.xq, st, optional));
-    float* h = static_cast<float*>(grow_scratch(g_scratch_gh, B.h, st, optional));
-    uint8_t* hq = static_cast<uint8_t*>(grow_scratch(g_scratch_ghq, B.hq, st, optional));
-    float* y = static_cast<float*>(grow_scratch(g_scratch_gy, B.y, st, optional));
-    if (!index || !xq || !h || !hq || !y) return pt ? 1 : -1;
-    const RowsIndex R = rows_index(index, P, E, pt ? pt : 2);
+    if (!grouped_scratch(grouped_bufs(L, n_used, n_tokens), st, pt != 0)) return pt ? 1 : -1;
+    uint8_t* xq = static_cast<uint8_t*>(g_scratch_gxq.p);
+    float* h = static_cast<float*>(g_scratch_gh.p);
+    uint8_t* hq = static_cast<uint8_t*>(g_scratch_ghq.p);
+    float* y = static_cast<float*>(g_scratch_gy.p);
+    const RowsIndex R = rows_index(g_scratch_goff.p, P, E, pt ? pt : 2);
     int *const off = R.off, *const pair_of = R.pair_of, *const pos_of = R.pos_of;
-    float *hs = nullptr, *shared = nullptr, *sgl = nullptr;
-    uint8_t *sxq = nullptr, *shq = nullptr;
-    if (L->shared_gate) {
-        hs = static_cast<float*>(grow_scratch(g_scratch_hs, sizeof(float) * (size_t)n_tokens * L->d_ff_shared, st));
-        shared = static_cast<float*>(grow_scratch(g_scratch_ys, sizeof(float) * (size_t)n_tokens * D, st));
-        if (!hs || !shared) return -1;
-    }
-    if (shared_dense(L, n_tokens)) {
-        sxq = static_cast<uint8_t*>(
-            grow_scratch(g_scratch_sxq, (size_t)n_tokens * dense_act_stride(L->qt_shared_gate, D), st));
-        shq = static_cast<uint8_t*>(
-            grow_scratch(g_scratch_shq, (size_t)n_tokens * dense_act_stride(L->qt_shared_down, L->d_ff_shared), st));
-        sgl = static_cast<float*>(grow_scratch(g_scratch_sgl, sizeof(float) * (size_t)n_tokens, st));
-        if (!sxq || !shq || !sgl) return -1;
-    }
+    Workspace ws;
+    LayerBufs sb;
+    if (shared_bufs(L, n_tokens, ws, st, sb)) return -1;
     std::unique_lock<std::mutex> side_lock(g_side_mu, std::defer_lock);
     hipEvent_t join = nullptr;
     if (shared_overlaps(L, n_tokens)) {
         side_lock.lock();
-        if (shared_expert_forked(L, d_x, n_tokens, hs, shared, sxq, shq, sgl, st)) return -1;
+        if (shared_expert_forked(L, d_x, n_tokens, sb.hs, sb.ys, sb.sxq, sb.shq, sb.sgl, st)) return -1;
         join = g_ev_join;
-    } else if (shared_expert(L, d_x, n_tokens, hs, shared, st, sxq, shq, sgl)) {
+    } else if (shared_expert(L, d_x, n_tokens, sb.hs, sb.ys, st, sb.sxq, sb.shq, sb.sgl)) {
         return -1;
     }
 
@@ -2283,9 +2291,9 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
         launch_grouped_down<false>(L->qt_down, KK_GDOWN, D, E, st, dn);
     }
     if (join && !ck(hipStreamWaitEvent(st, join, 0), "join the shared expert")) return -1;
-    CombineArgs cb{y, pos_of, d_w, shared, d_resid, d_out, n_used, D};
+    CombineArgs cb{y, pos_of, d_w, sb.ys, d_resid, d_out, n_used, D};
     const bool v4 = D % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_out) | reinterpret_cast<uintptr_t>(d_resid) |
-                                    reinterpret_cast<uintptr_t>(shared)) & 15) == 0;
+                                    reinterpret_cast<uintptr_t>(sb.ys)) & 15) == 0;
     if (v4)
         hipLaunchKernelGGL(k_combine<4>, dim3((unsigned)((D + 4 * kThreads - 1) / (4 * kThreads)), (unsigned)n_tokens),
                            dim3(kThreads), 0, st, cb);
@@ -2324,11 +2332,22 @@ SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const f
     if (n_tokens == 0) return 0;
     ++g_layer_calls;
     g_lookups += (unsigned long long)n_tokens * n_used;
+    hipStream_t st = pick_stream(stream);
     if (prefill_takes_rows(layer, (size_t)n_tokens * n_used)) {
-        const int rc = moe_layer_rows(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, pick_stream(stream));
+        const int rc = moe_layer_rows(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, st);
+        if (rc == 0 && !stream_capturing(st)) {
+            // room for the smaller batches that take the other kernels in one piece: one captured
+            // later could not grow it (this call does without it)
+            const int n = largest_other(n_tokens, [&](int t) {
+                return prefill_takes_rows(layer, (size_t)t * n_used) && rows_layer_ok(layer, n_used, t);
+            });
+            Workspace ws;
+            LayerBufs b;
+            (void)(grouped_scratch(grouped_bufs(layer, n_used, n), st) && !shared_bufs(layer, n, ws, st, b));
+        }
         if (rc <= 0) return rc;
     }
-    return moe_grouped_on(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, 0, pick_stream(stream));
+    return moe_grouped_on(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, 0, st);
 }
 
 SABAH_API int sabah_moe_route(const float* d_logits, int n_tokens, int n_experts, int n_used, int norm_w,

@@ -333,6 +333,31 @@ def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
         assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
 
 
+def test_a_smaller_fixed_shape_prefill_is_captured_after_a_grouped_rows_one(hip_rt):
+    """4,096 experts: 90,000 pairs take k_grouped_rows in runs of 65,536, and the
+    80,000 pairs captured after them the fixed-shape kernels, in one piece."""
+    from sabah.runtime.bank import ExpertBank
+    from sabah.runtime.executor import MoEExecutor
+    E, K, D, F, tokens, small = 4096, 10, 512, 256, 9000, 8000
+    rng = np.random.default_rng(42)
+    bank = ExpertBank(1, E, D, F, {"gate": IQ3_S, "up": IQ3_S, "down": Q6_K}, device="cuda:0")
+    bank.fill_synthetic(seed=5)
+    ex = MoEExecutor(bank, max_used=K)
+    x = T(rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    big = ex.run_prefill_layer(0, x, ids, w)
+    out = torch.empty_like(x[:small])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ex.run_prefill_layer(0, x[:small], ids[:small], w[:small], out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_bits_equal(out.cpu().numpy(), big[:small].cpu().numpy(), "replayed prefill")
+
+
 # q8 rows past 2 GiB and past 2^21 chunks in all: in the general form with one x row
 # per slot (450,000 rows of 4,864 bytes) and in the fixed-shape form (900,000 of 2,464)
 @pytest.mark.parametrize("qt,k,tokens,K,slot_rows", [(Q8_0, 4096, 45000, 10, True), (Q4_K, 2048, 45000, 20, False)])
