@@ -1994,8 +1994,8 @@ static bool shared_overlaps(const sabah_moe_layer_desc* L, int n_tokens) { retur
 // A layer over many tokens in the general grouped form (k_grouped_rows), for
 // sabah_moe_layer and the chain.
 // ---------------------------------------------------------------------------
-// A batch of more than kRowsMaxPairs pairs runs in runs of tokens, so the
-// scratch stays bounded.
+// A batch of more than kRowsMaxPairs pairs runs in runs of tokens, and its
+// scratch is one run's.
 constexpr size_t kRowsMaxPairs = 65536;
 static int rows_run(int n_used, int n_tokens) { return std::min(n_tokens, std::max(1, (int)(kRowsMaxPairs / n_used))); }
 static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
@@ -2008,7 +2008,7 @@ static bool rows_layer_ok(const sabah_moe_layer_desc* L, int n_used, int n_token
 }
 static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                           int n_used, int n_tokens, float* d_out, const float* d_resid, int pt, hipStream_t st);
-static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, hipStream_t st);
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st);
 // the largest batch below n_tokens that is not one of `takes` (which is true from
 // some size on, and of n_tokens, and never of one token)
 template <typename F>
@@ -2026,7 +2026,7 @@ static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const
     if (!rows_layer_ok(L, n_used, n_tokens)) return 1;
     const int run = rows_run(n_used, n_tokens);
     const int pt = rows_tiles((size_t)run * n_used, L->n_experts, L->d_ff, L->qt_gate == QT_Q8_0);
-    if (!grouped_layer_ready(L, n_used, run, st)) return 1;
+    if (!grouped_layer_ready(L, n_used, run, pt, st)) return 1;
     for (int t = 0; t < n_tokens; t += run) {
         const size_t td = (size_t)t * L->d_model, tk = (size_t)t * n_used;
         const int rc = moe_grouped_on(L, d_x + td, d_ids + tk, d_w + tk, n_used, std::min(run, n_tokens - t), d_out + td,
@@ -2039,14 +2039,18 @@ static int moe_layer_rows(const sabah_moe_layer_desc* L, const float* d_x, const
 static int moe_layer_on(const sabah_moe_layer_desc* L, const float* d_x, const int32_t* d_ids, const float* d_w,
                         int n_used, int n_tokens, float* d_out, const float* d_resid, Workspace& ws, hipStream_t st) {
     const int D = L->d_model, F = L->d_ff;
-    // sized for the token-major form also where the grouped one runs: a smaller call
-    // captured later may take the former, and cannot grow them
     LayerBufs b;
-    if (layer_bufs(L, n_used, n_tokens, ws, st, b)) return -1;
     if (!ws.arena) {
         const int rc = moe_layer_rows(L, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, st);
+        if (rc == 0 && !stream_capturing(st)) {
+            // room for the smaller batches that take the token-major kernels: one captured later
+            // could not grow it (this call does without it)
+            const int n = largest_other(n_tokens, [&](int t) { return rows_layer_ok(L, n_used, t); });
+            (void)layer_bufs(L, n_used, n, ws, st, b);
+        }
         if (rc <= 0) return rc;
     }
+    if (layer_bufs(L, n_used, n_tokens, ws, st, b)) return -1;
     std::unique_lock<std::mutex> side_lock(g_side_mu, std::defer_lock);
     hipEvent_t join = nullptr;
     if (shared_overlaps(L, n_tokens)) {
@@ -2172,17 +2176,15 @@ static bool grouped_shape_ok(const sabah_moe_layer_desc* L) {
 
 // Scratch of a group-major layer.  pt = 0: the fixed-shape kernels' (the
 // pairs' x rows quantised in group order); pt = 2, 4: k_grouped_rows with items of pt
-// 16-pair tiles (one q8 row per token; xq is sized for the pairs all the same,
-// so a smaller call that takes the other kernels finds its room in a capture).  The index
-// is sized for two-tile items, the more of the two, so that no smaller batch needs more than
-// a larger one.
+// 16-pair tiles (one q8 row of x per token).  The index is sized for two-tile items, the
+// more of the two, so that no smaller batch needs more than a larger one.
 struct GroupedBufs {
     size_t index, xq, h, hq, y;
 };
-static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens) {
+static GroupedBufs grouped_bufs(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt) {
     const size_t P = (size_t)n_tokens * n_used;
     return {rows_index_bytes(P, L->n_experts, 2),
-            ActLayout(L->d_model, act_type(L->qt_gate)).bytes * P, sizeof(float) * P * L->d_ff,
+            ActLayout(L->d_model, act_type(L->qt_gate)).bytes * (pt ? (size_t)n_tokens : P), sizeof(float) * P * L->d_ff,
             ActLayout(L->d_ff, act_type(L->qt_down)).bytes * P, sizeof(float) * P * L->d_model};
 }
 // false inside a capture for which the scratch would have to grow
@@ -2197,8 +2199,8 @@ static bool grouped_scratch(const GroupedBufs& B, hipStream_t st, bool optional 
            grow_scratch(g_scratch_gy, B.y, st, optional);
 }
 
-static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, hipStream_t st) {
-    return grouped_scratch_ready(grouped_bufs(L, n_used, n_tokens), st);
+static bool grouped_layer_ready(const sabah_moe_layer_desc* L, int n_used, int n_tokens, int pt, hipStream_t st) {
+    return grouped_scratch_ready(grouped_bufs(L, n_used, n_tokens, pt), st);
 }
 
 // 0 done, -1 error, 1 (pt > 0 only) nothing launched: no memory for the scratch
@@ -2208,7 +2210,7 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
     const size_t P = (size_t)n_tokens * n_used;
     const int xq_stride = (int)ActLayout(D, act_type(L->qt_gate)).bytes;
     const int hq_stride = (int)ActLayout(F, act_type(L->qt_down)).bytes;
-    if (!grouped_scratch(grouped_bufs(L, n_used, n_tokens), st, pt != 0)) return pt ? 1 : -1;
+    if (!grouped_scratch(grouped_bufs(L, n_used, n_tokens, pt), st, pt != 0)) return pt ? 1 : -1;
     uint8_t* xq = static_cast<uint8_t*>(g_scratch_gxq.p);
     float* h = static_cast<float*>(g_scratch_gh.p);
     uint8_t* hq = static_cast<uint8_t*>(g_scratch_ghq.p);
@@ -2336,14 +2338,13 @@ SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const f
     if (prefill_takes_rows(layer, (size_t)n_tokens * n_used)) {
         const int rc = moe_layer_rows(layer, d_x, d_ids, d_w, n_used, n_tokens, d_out, d_resid, st);
         if (rc == 0 && !stream_capturing(st)) {
-            // room for the smaller batches that take the other kernels in one piece: one captured
-            // later could not grow it (this call does without it)
+            // room for the smaller batches that take the other kernels, as in moe_layer_on
             const int n = largest_other(n_tokens, [&](int t) {
                 return prefill_takes_rows(layer, (size_t)t * n_used) && rows_layer_ok(layer, n_used, t);
             });
             Workspace ws;
             LayerBufs b;
-            (void)(grouped_scratch(grouped_bufs(layer, n_used, n), st) && !shared_bufs(layer, n, ws, st, b));
+            (void)(grouped_scratch(grouped_bufs(layer, n_used, n, 0), st) && !shared_bufs(layer, n, ws, st, b));
         }
         if (rc <= 0) return rc;
     }

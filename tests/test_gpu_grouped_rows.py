@@ -333,6 +333,30 @@ def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
         assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
 
 
+def test_a_large_layers_scratch_is_one_runs(hip_rt):
+    """200,000 pairs run in four runs of tokens (three of 65,536 pairs and a rest):
+    the scratch is one run's (h of the whole batch alone would be 3.3 GB), and every
+    run's tokens are the token-major layer's."""
+    from sabah.runtime import rt
+    E, K, D, F, tokens = 6, 2, 64, 4096, 100000
+    rng = np.random.default_rng(41)
+    banks = [T(bank_bytes(rng, Q8_0, E, rows, k)) for rows, k in ((F, D), (F, D), (D, F))]
+    desc = rt.MoeLayerDesc()
+    desc.gate, desc.up, desc.down = (b.data_ptr() for b in banks)
+    desc.qt_gate = desc.qt_up = desc.qt_down = Q8_0
+    desc.d_model, desc.d_ff, desc.n_experts = D, F, E
+    x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    w = T(rng.random((tokens, K)).astype(np.float32))
+    before = hip_rt.snapshot()["scratch_bytes"]
+    got = layer(hip_rt, "sabah_moe_layer", desc, x, ids, w, x)
+    assert hip_rt.snapshot()["scratch_bytes"] - before < 2.5e9
+    for t in (0, 32768 - 60, 2 * 32768 - 60, 3 * 32768 - 60, tokens - 120):
+        s = slice(t, t + 120)                     # across the runs' ends
+        want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, *(a[s].contiguous() for a in (x, ids, w, x)))
+        assert_bits_equal(got[s], want, "tokens from %d" % t)
+
+
 def test_a_smaller_fixed_shape_prefill_is_captured_after_a_grouped_rows_one(hip_rt):
     """4,096 experts: 90,000 pairs take k_grouped_rows in runs of 65,536, and the
     80,000 pairs captured after them the fixed-shape kernels, in one piece."""
