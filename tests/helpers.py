@@ -52,6 +52,31 @@ def assert_bits_equal(got, want, what=""):
             what, bad.size, g.size, int((gf[bad] == 0xFFFFFFFF).sum()), int((wf[bad] == 0xFFFFFFFF).sum()), first))
 
 
+def token_major_layer(ex, layer, x, ids, w, resid=None):
+    """A layer of executor ex by the token-major kernels whatever the batch:
+    sabah_moe_layer_noalloc, which never groups, over as many tokens at a time as
+    its 8 MiB of scratch hold."""
+    import ctypes
+
+    import torch
+    from sabah.runtime import rt
+    desc = ex.bank.layer_desc(layer, ex.shared)
+    K = ids.shape[1]
+    per_token = 6 * K * ex.ff + (8 * ex.d_model + 8 * ex.shared.d_ff if ex.shared is not None else 0)
+    step = max(1, (7 << 20) // per_token)
+    out = torch.full_like(x, float("nan"))
+    for t in range(0, x.shape[0], step):
+        a = [v[t:t + step].contiguous() for v in (x, ids, w)]
+        r = None if resid is None else resid[t:t + step].contiguous()
+        o = torch.empty_like(a[0])
+        rt.check(rt.lib().sabah_moe_layer_noalloc(
+            ctypes.byref(desc), *(ctypes.c_void_p(v.data_ptr()) for v in a), K, a[0].shape[0],
+            ctypes.c_void_p(o.data_ptr()), ctypes.c_void_p(r.data_ptr()) if r is not None else None,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "moe_layer_noalloc")
+        out[t:t + step] = o
+    return out
+
+
 def f16(x: float) -> bytes:
     return np.array([x], np.float16).tobytes()
 

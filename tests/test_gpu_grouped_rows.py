@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_bits_equal, assert_parity, random_blocks
+from helpers import assert_bits_equal, assert_parity, random_blocks, token_major_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -304,6 +304,99 @@ def test_grouped_layer_is_bit_identical_to_token_major(hip_rt, qtg, qtd, D, F, t
         assert_bits_equal(out.cpu().numpy(), want, "replayed layer")
 
 
+def typed_executor(rng, qtg, qtd, E, D, F, K, shared=None):
+    """An executor over one layer of random valid blocks."""
+    from sabah.runtime.bank import ExpertBank
+    from sabah.runtime.executor import MoEExecutor
+    bank = ExpertBank(1, E, D, F, {"gate": qtg, "up": qtg, "down": qtd}, device="cuda:0")
+    for role, qt, rows, k in (("gate", qtg, F, D), ("up", qtg, F, D), ("down", qtd, D, F)):
+        bank.load(0, role, bank_bytes(rng, qt, E, rows, k))
+    return MoEExecutor(bank, max_used=K, shared=shared)
+
+
+def layer_inputs(rng, E, D, K, tokens):
+    ids = np.argsort(rng.random((tokens, E)), axis=1)[:, :K].astype(np.int32)
+    ids[1, 1] = ids[1, 0]                            # a duplicate
+    return (T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32)), T(ids),
+            T(rng.random((tokens, K)).astype(np.float32)))
+
+
+# four-tile items: 602 pairs over 6 experts (at least 24 each on average; items of 64
+# and a rest that ends inside a tile) at d_ff 4608 (72 row tiles x 15 items >= 1,024)
+@pytest.mark.parametrize("qtg,qtd,D", [(Q4_K, Q6_K, 512), (Q6_K, Q4_K, 256), (Q4_K, Q8_0, 256), (Q5_K, IQ4_XS, 256),
+                                       (IQ3_S, IQ3_S, 256), (IQ3_XXS, IQ4_NL, 512), (IQ4_XS, Q5_K, 256),
+                                       (IQ4_NL, IQ3_XXS, 352)])
+def test_grouped_layer_of_four_tile_items(hip_rt, qtg, qtd, D):
+    E, K, F, tokens = 6, 2, 4608, 301
+    rng = np.random.default_rng(1000 * qtg + qtd)
+    ex = typed_executor(rng, qtg, qtd, E, D, F, K)
+    x, ids, w = layer_inputs(rng, E, D, K, tokens)
+    for resid in (None, x):
+        got = ex.run_layer(0, x, ids, w, resid=resid)
+        want = token_major_layer(ex, 0, x, ids, w, resid)
+        assert_bits_equal(got.cpu().numpy(), want.cpu().numpy(), "layer %d/%d" % (qtg, qtd))
+
+
+# sabah_moe_prefill_layer's batches on k_grouped_rows: from 10 pairs per expert and 512 in
+# all (20 and 4,096 with an IQ3_S matrix), in two- and four-tile items (40 experts, 1,600 pairs)
+@pytest.mark.parametrize("qtg,qtd,E,D,F,K,tokens", [
+    (Q4_K, Q6_K, 6, 512, 256, 2, 256), (Q6_K, Q4_K, 51, 1024, 512, 3, 171), (Q4_K, Q6_K, 40, 512, 1024, 4, 401),
+    (Q6_K, Q6_K, 40, 512, 1024, 4, 400), (Q4_K, Q4_K, 40, 2048, 1024, 4, 400), (IQ3_S, Q4_K, 200, 512, 512, 8, 513),
+    (Q4_K, IQ3_S, 40, 512, 1024, 4, 1025), (IQ3_S, IQ3_S, 40, 512, 1024, 4, 1025)])
+def test_prefill_layer_on_grouped_rows(hip_rt, qtg, qtd, E, D, F, K, tokens):
+    rng = np.random.default_rng(100 * qtg + qtd + tokens)
+    ex = typed_executor(rng, qtg, qtd, E, D, F, K)
+    x, ids, w = layer_inputs(rng, E, D, K, tokens)
+    want = token_major_layer(ex, 0, x, ids, w, x).cpu().numpy()
+    hip_rt.check(hip_rt.lib().sabah_rt_set_kernel_timing(1), "timing on")
+    try:
+        grouped_launches(hip_rt)
+        got = ex.run_prefill_layer(0, x, ids, w, resid=x)
+        torch.cuda.synchronize()
+        assert grouped_launches(hip_rt) == 3         # the grouping, x's rows and gate/up (the fixed-shape form times one)
+    finally:
+        hip_rt.check(hip_rt.lib().sabah_rt_set_kernel_timing(0), "timing off")
+    assert_bits_equal(got.cpu().numpy(), want, "prefill %d/%d" % (qtg, qtd))
+
+
+# k_group_pairs with its ids in 8 or 16 registers a thread, and read again: at most 8,192
+# and 16,384 pairs, and more
+@pytest.mark.parametrize("tokens", [2730, 2731, 5461, 5462, 7001])
+def test_grouping_of_many_pairs(hip_rt, grouping, tokens):
+    E, K, rows, k = 37, 3, 17, 256
+    rng = np.random.default_rng(tokens)
+    bank = T(bank_bytes(rng, IQ4_XS, E, rows, k))
+    ids = rng.integers(0, E, (tokens, K)).astype(np.int32)
+    ids[tokens - 1, 2] = E                           # a bad id, in the last pair
+    x = T(rng.standard_normal((tokens, 1, k)).astype(np.float32))
+    grouping(NEVER)
+    tok = mmid(hip_rt, bank, IQ4_XS, rows, k, E, x, T(ids), grouped=False)
+    assert hip_rt.lib().sabah_rt_check_errors() == -1
+    grouping(ALWAYS)
+    got = mmid(hip_rt, bank, IQ4_XS, rows, k, E, x, T(ids), grouped=True)
+    assert hip_rt.lib().sabah_rt_check_errors() == -1
+    assert np.isnan(got[tokens - 1, 2]).all() and np.isnan(tok[tokens - 1, 2]).all()
+    got[tokens - 1, 2] = tok[tokens - 1, 2] = 0
+    assert_bits_equal(got, tok, "%d pairs" % (tokens * K))
+
+
+def test_runs_of_tokens_beside_a_gated_shared_expert(hip_rt):
+    """70,010 pairs in two runs of tokens, each with the shared expert on the side
+    stream beside it and the residual."""
+    from sabah.runtime.bank import DenseExpert
+    E, D, F, K, tokens = 12, 256, 256, 10, 7001
+    rng = np.random.default_rng(71)
+    shared = DenseExpert(D, 256, Q8_0, device="cuda:0")
+    for role in ("gate", "up", "down"):
+        shared.load(role, random_blocks(rng, Q8_0, 256, 256))
+    shared.set_gate((0.05 * rng.standard_normal(D)).astype(np.float32))
+    ex = typed_executor(rng, Q5_K, Q8_0, E, D, F, K, shared)
+    x, ids, w = layer_inputs(rng, E, D, K, tokens)
+    got = ex.run_layer(0, x, ids, w, resid=x)
+    want = token_major_layer(ex, 0, x, ids, w, x)
+    assert_bits_equal(got.cpu().numpy(), want.cpu().numpy(), "layer")
+
+
 def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
     """An eager call that runs group-major leaves room for a smaller, token-major
     call of the same layer inside a capture, which cannot allocate."""
@@ -318,7 +411,11 @@ def test_a_smaller_token_major_layer_is_captured_after_a_grouped_one(hip_rt):
     x = T(0.05 * rng.standard_normal((tokens, D)).astype(np.float32))
     ids = T(np.stack([rng.choice(E, K, replace=False) for _ in range(tokens)]).astype(np.int32))
     w = T(rng.random((tokens, K)).astype(np.float32))
-    layer(hip_rt, "sabah_moe_layer", desc, x, ids, w)
+    got = layer(hip_rt, "sabah_moe_layer", desc, x, ids, w)
+    for t in range(0, tokens, 100):
+        s = slice(t, t + 100)
+        want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x[s].contiguous(), ids[s].contiguous(), w[s].contiguous())
+        assert_bits_equal(got[s], want, "the eager layer, tokens from %d" % t)
     want = layer(hip_rt, "sabah_moe_layer_noalloc", desc, x[:small], ids[:small], w[:small])
     out = torch.empty_like(x[:small])
     graph = torch.cuda.CUDAGraph()

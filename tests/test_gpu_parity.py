@@ -13,7 +13,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_parity, random_blocks, unfused_rounding_row, assert_bits_equal, q8_1_tie_row
+from helpers import (assert_bits_equal, assert_parity, q8_1_tie_row, random_blocks, token_major_layer,
+                     unfused_rounding_row)
 
 pytestmark = pytest.mark.gpu
 
@@ -364,9 +365,10 @@ def test_moe_block_single_token_q8_0(hip_rt, orc):
 # iq3xxs_iq4nl_artifact_shape: the quant mix of the reference's shipped block
 # (IQ3_XXS gate/up, IQ4_NL down; results/bench_moe_blk0_iq3s.json) at its
 # inferred shape, d_model 2560 and expert d_ff 640 (REPORT.md:345-347)
-# iq3s_t32: 32 tokens, so gate/up and down run grown multi-pass row tiles and
-# down reads h quantised once per (token, slot) row (q8_K rows); q8_0_t4_hq and
-# iq4nl_down_t3_hq take that path with q8_0 rows (Q8_0 / IQ4_NL down, d_ff 768)
+# iq3s_t32: 32 tokens, so the token-major gate/up and down run grown multi-pass row
+# tiles and down reads h quantised once per (token, slot) row (q8_K rows); q8_0_t4_hq and
+# iq4nl_down_t3_hq take that path with q8_0 rows (Q8_0 / IQ4_NL down, d_ff 768).
+# sabah_moe_layer groups the 32-token batches; the token-major layer is compared as well
 @pytest.mark.parametrize("name", ["q4k_e128_top8", "mixed_t32_q4k_q6k_shared", "iq3s_small", "iq3s_t32",
                                   "iq3xxs_iq4nl_artifact_shape", "iq4xs_small", "iq2s_iq3s_mix", "q8_0_t4_hq",
                                   "iq4nl_down_t3_hq", "q2_0_decode", "q2_0_down_t3_hq", "q2_0_partial_units",
@@ -443,6 +445,7 @@ def test_moe_layer_matches_oracle(hip_rt, orc, name):
     sh = None if sh_raw is None else (sh_raw["gate"], sh_raw["up"], sh_raw["down"], (Q8_0,) * 3)
     want = orc.moe_layer(raws[(0, "gate")], raws[(0, "up")], raws[(0, "down")], qts, x, ids, w, shared=sh)
     assert_parity(out.cpu().numpy(), want, name)
+    assert_bits_equal(token_major_layer(ex, 0, T(x), T(ids), T(w)).cpu().numpy(), out.cpu().numpy(), name)
     if name.startswith("q2_0") or name.startswith("q5_1"):
         assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
 

@@ -3,9 +3,10 @@
 sabah_moe_prefill_layer groups the (token, slot) pairs by expert on the
 device and applies each expert's rows to all of its pairs with int8 MFMA
 (IQ3_S, Q4_K and Q6_K weights; the K formats' bsum side terms on fp32 MFMA).
-Bar: bit-identical to the token-major sabah_moe_layer on the same inputs
-(same integer block sums, same fp32 order), and within max_rel <= 1e-3,
-cosine >= 0.99999 of the oracle's layer.
+Bar: bit-identical to the token-major layer on the same inputs (same integer
+block sums, same fp32 order; helpers.token_major_layer, since sabah_moe_layer
+itself groups many of these batches), as is sabah_moe_layer, and within max_rel
+<= 1e-3, cosine >= 0.99999 of the oracle's layer.
 """
 from __future__ import annotations
 
@@ -15,7 +16,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_parity, random_blocks
+from helpers import assert_parity, random_blocks, token_major_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -76,8 +77,10 @@ def test_prefill_layer_is_the_token_major_layer(hip_rt, orc, case, E, D, F, Tn, 
     x = rng.standard_normal((Tn, D)).astype(np.float32)
     ex = MoEExecutor(bank, max_used=K)
     got = ex.run_prefill_layer(0, T(x), T(ids), T(w))
-    ref = ex.run_layer(0, T(x), T(ids), T(w))
+    ref = token_major_layer(ex, 0, T(x), T(ids), T(w))
+    also = ex.run_layer(0, T(x), T(ids), T(w))
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.equal(got, ref), "grouped layer differs from the token-major layer (%s)" % case
     want = orc.moe_layer(raws["gate"], raws["up"], raws["down"], (IQ3_S,) * 3, x, ids, w)
     assert_parity(got.cpu().numpy(), want, "prefill %s" % case)
@@ -103,8 +106,10 @@ def test_prefill_layer_with_shared_expert_and_residual(hip_rt, orc, gated):
     ex = MoEExecutor(bank, max_used=K, shared=shared)
     xd = T(x)
     got = ex.run_prefill_layer(0, xd, T(ids), T(w), resid=xd)
-    ref = ex.run_layer(0, xd, T(ids), T(w), resid=xd)
+    ref = token_major_layer(ex, 0, xd, T(ids), T(w), resid=xd)
+    also = ex.run_layer(0, xd, T(ids), T(w), resid=xd)
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.equal(got, ref)
     y = orc.moe_layer(raws["gate"], raws["up"], raws["down"], (IQ3_S,) * 3, x, ids, w,
                       shared=(sh_raw["gate"], sh_raw["up"], sh_raw["down"], (Q8_0,) * 3, row))
@@ -168,8 +173,10 @@ def test_prefill_layer_full_size_matches_token_major(hip_rt, orc):
     x = rng.standard_normal((Tn, D)).astype(np.float32)
     ex = MoEExecutor(bank, max_used=K)
     got = ex.run_prefill_layer(0, T(x), T(ids), T(w))
-    ref = ex.run_layer(0, T(x), T(ids), T(w))
+    ref = token_major_layer(ex, 0, T(x), T(ids), T(w))
+    also = ex.run_layer(0, T(x), T(ids), T(w))
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.isfinite(got).all()
     assert torch.equal(got, ref)
 
@@ -187,8 +194,10 @@ def test_grouped_k_formats_are_the_token_major_layer(hip_rt, orc, qg, qd, case):
     x = rng.standard_normal((Tn, D)).astype(np.float32)
     ex = MoEExecutor(bank, max_used=K)
     got = ex.run_prefill_layer(0, T(x), T(ids), T(w))
-    ref = ex.run_layer(0, T(x), T(ids), T(w))
+    ref = token_major_layer(ex, 0, T(x), T(ids), T(w))
+    also = ex.run_layer(0, T(x), T(ids), T(w))
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.equal(got, ref), "grouped %d/%d layer differs from the token-major layer (%s)" % (qg, qd, case)
     want = orc.moe_layer(raws["gate"], raws["up"], raws["down"], (qg, qg, qd), x, ids, w)
     assert_parity(got.cpu().numpy(), want, "prefill %d/%d %s" % (qg, qd, case))
@@ -207,8 +216,10 @@ def test_grouped_k_formats_random_blocks(hip_rt, orc, qg, qd):
     x = rng.standard_normal((Tn, D)).astype(np.float32)
     ex = MoEExecutor(bank, max_used=K)
     got = ex.run_prefill_layer(0, T(x), T(ids), T(w))
-    ref = ex.run_layer(0, T(x), T(ids), T(w))
+    ref = token_major_layer(ex, 0, T(x), T(ids), T(w))
+    also = ex.run_layer(0, T(x), T(ids), T(w))
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.isfinite(ref).all()
     assert torch.equal(got, ref)
 
@@ -231,7 +242,9 @@ def test_grouped_mixed_layer_full_size_matches_token_major(hip_rt, orc):
     ex = MoEExecutor(bank, max_used=K, shared=shared)
     xd = T(x)
     got = ex.run_prefill_layer(0, xd, T(ids), T(w), resid=xd)
-    ref = ex.run_layer(0, xd, T(ids), T(w), resid=xd)
+    ref = token_major_layer(ex, 0, xd, T(ids), T(w), resid=xd)
+    also = ex.run_layer(0, xd, T(ids), T(w), resid=xd)
     torch.cuda.synchronize()
+    assert torch.equal(also, ref)
     assert torch.isfinite(got).all()
     assert torch.equal(got, ref)
