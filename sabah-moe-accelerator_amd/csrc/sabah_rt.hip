@@ -1160,31 +1160,33 @@ static int rows_groups(int qt, int pt, int rows, size_t items) {
     const int tiles = (rows + 2 * kRowsTile - 1) / (2 * kRowsTile);
     return qt != QT_Q8_0 && pt == 2 && tiles * 2 * kRowsTile <= rows + rows / 8 && (size_t)tiles * items >= 1024 ? 2 : 1;
 }
+// The forms that are built: two row groups outside gate/up only with two tiles and not of
+// Q8_0 (rows_groups), and four tiles of Q8_0 gate/up not at all (rows_tiles)
+template <int QT, int G, int MODE>
+static void launch_rows_qt(int kind, int pt, dim3 grid, const GroupedRowsArgs& a, hipStream_t st, hipEvent_t done) {
+    constexpr bool SWIGLU = MODE == kRowsSwiglu;
+    if constexpr (QT != QT_Q8_0 || G == 1 || SWIGLU) {
+        if constexpr (G == 1 || (SWIGLU && QT != QT_Q8_0))
+            if (pt == 4)
+                return launch_kernel_done(done, kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a);
+        launch_kernel_done(done, kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);
+    }
+}
 template <int G, int MODE>
 static void launch_rows_g(int qt, int kind, int pt, size_t items, const GroupedRowsArgs& a, hipStream_t st,
                           hipEvent_t done) {
     const int tile = MODE == kRowsSwiglu ? kRowsTile : G * kRowsTile;
     const dim3 grid((unsigned)((a.rows + tile - 1) / tile), (unsigned)items);
-#define SB_ROWS(QT)                                                                                           \
-    case QT:                                                                                                   \
-        if constexpr (G == 1 || (MODE == kRowsSwiglu && QT != QT_Q8_0))                                        \
-            if (pt == 4) {                                                                                     \
-                launch_kernel_done(done, kind, k_grouped_rows<QT, G, 4, MODE>, grid, dim3(kThreads), 0, st, a);    \
-                break;                                                                                         \
-            }                                                                                                  \
-        launch_kernel_done(done, kind, k_grouped_rows<QT, G, 2, MODE>, grid, dim3(kThreads), 0, st, a);        \
-        break;
     switch (qt) {
-    SB_ROWS(QT_Q8_0)
-    SB_ROWS(QT_Q4_K)
-    SB_ROWS(QT_Q5_K)
-    SB_ROWS(QT_Q6_K)
-    SB_ROWS(QT_IQ3_S)
-    SB_ROWS(QT_IQ3_XXS)
-    SB_ROWS(QT_IQ4_NL)
-    SB_ROWS(QT_IQ4_XS)
+    case QT_Q8_0: return launch_rows_qt<QT_Q8_0, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_Q4_K: return launch_rows_qt<QT_Q4_K, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_Q5_K: return launch_rows_qt<QT_Q5_K, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_Q6_K: return launch_rows_qt<QT_Q6_K, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_IQ3_S: return launch_rows_qt<QT_IQ3_S, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_IQ3_XXS: return launch_rows_qt<QT_IQ3_XXS, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_IQ4_NL: return launch_rows_qt<QT_IQ4_NL, G, MODE>(kind, pt, grid, a, st, done);
+    case QT_IQ4_XS: return launch_rows_qt<QT_IQ4_XS, G, MODE>(kind, pt, grid, a, st, done);
     }
-#undef SB_ROWS
 }
 // done: recorded as the kernel ends (or null)
 template <int MODE>
@@ -1206,24 +1208,36 @@ static void launch_rows(int qt, int kind, int pt, size_t items, const GroupedRow
 //            IQ4_XS 130 - 230 / 110 - 140 / 85 - 130 / 32; IQ3_XXS gate 290 / 170 / 130 / 110, IQ4_NL down 970 / 245 / 145 / 56
 // e.g. (token-major / grouped, us) an IQ4_XS layer at 32 tokens, top-10 of 512: 374 / 218; Q8_0
 // at 16 tokens, top-2 of 8: 51 / 41, at 8: 32 / 41.
+//
+// And no fewer than floor + chain k / 1024 pairs (2 M weights again): with few experts the launch
+// does not fill the chip, and its time is that of k / 256 dependent steps however few
+// the pairs.  Measured (MUL_MAT_ID over 8 experts, token-major / grouped, us): IQ4_XS 640 x 2560 at
+// 54 pairs 15.7 / 26.1, at 94 26.6 / 26.1; Q8_0 768 x 2048 at 56 16.8 / 24.6, at 90 27.5 / 24.4; IQ3_XXS
+// 4096 x 14336 at 8 54 / 90, at 14 90 / 89.  Of 5,700 calls (8 formats, 9 shapes, 8 - 512 experts, uniform and Zipf
+// routing, 0.6 - 4 times the line) the first line alone groups 4,356, 144 of them more than 3 % slower
+// than token-major (the worst at 0.60 of its speed); both lines group 4,214, 35 of them slower (0.80).
 struct RowsCost {
-    int base, per16;
+    int base, per16, floor, chain;
 };
 static RowsCost rows_cost(int qt, bool layer) {
     switch (qt) {
-    case QT_Q8_0: return layer ? RowsCost{24, 9} : RowsCost{36, 14};
-    case QT_Q6_K: return layer ? RowsCost{24, 9} : RowsCost{36, 12};
-    case QT_Q4_K: return layer ? RowsCost{28, 16} : RowsCost{48, 18};
-    case QT_Q5_K: return layer ? RowsCost{24, 10} : RowsCost{36, 14};
-    case QT_IQ3_S: return layer ? RowsCost{44, 28} : RowsCost{60, 24};
-    case QT_IQ3_XXS: return layer ? RowsCost{40, 11} : RowsCost{80, 10};
-    case QT_IQ4_XS: return layer ? RowsCost{32, 7} : RowsCost{36, 9};
-    default: return layer ? RowsCost{44, 28} : RowsCost{44, 29};       // IQ4_NL
+    case QT_Q8_0: return layer ? RowsCost{24, 9, 12, 10} : RowsCost{36, 14, 28, 14};
+    case QT_Q6_K: return layer ? RowsCost{24, 9, 4, 12} : RowsCost{36, 12, 0, 18};
+    case QT_Q4_K: return layer ? RowsCost{28, 16, 0, 0} : RowsCost{48, 18, 56, 10};
+    case QT_Q5_K: return layer ? RowsCost{24, 10, 0, 0} : RowsCost{36, 14, 28, 14};
+    case QT_IQ3_S: return layer ? RowsCost{44, 28, 0, 0} : RowsCost{60, 24, 36, 16};
+    case QT_IQ3_XXS: return layer ? RowsCost{40, 11, 0, 0} : RowsCost{80, 10, 4, 24};
+    case QT_IQ4_XS: return layer ? RowsCost{32, 7, 0, 0} : RowsCost{36, 9, 28, 14};
+    default: return layer ? RowsCost{44, 28, 0, 0} : RowsCost{44, 29, 32, 14};       // IQ4_NL
     }
 }
 static bool rows_worth_it(int qt, bool layer, size_t pairs, int n_experts, int rows, int k) {
     const RowsCost c = rows_cost(qt, layer);
-    return 16.0 * (double)pairs >= 16.0 * c.base * (double)(1 << 21) / ((double)rows * k) + (double)c.per16 * n_experts;
+    const double m = (double)(1 << 21) / ((double)rows * k);
+    // past 8,192 the token-major kernels' own time per pair rises with k as well, but for
+    // IQ3_XXS's (IQ4_XS 4096 x 14336 at 6 pairs: 118 / 74 us)
+    const int kc = qt == QT_IQ3_XXS ? k : std::min(k, 8192);
+    return (double)pairs >= std::max(c.base * m + c.per16 * n_experts / 16.0, (c.floor + c.chain * kc / 1024.0) * m);
 }
 static bool mmid_rows_ok(int qt, bool packed, const uint8_t* bank, size_t expert_stride, size_t ids_id_stride,
                          size_t ids_token_stride, size_t x_id_stride, size_t x_token_stride, int x_rows, int n_ids,
@@ -2312,9 +2326,16 @@ static int moe_grouped_on(const sabah_moe_layer_desc* L, const float* d_x, const
 // 128 131 / 135 at 6, 190 / 159 at 16, 795 / 500 at 125; Q4_K / IQ3_S 146 / 150 at
 // 16, 214 / 199 at 32; IQ3_S 467 / 507 at 10, 683 / 598 at 20, 572 / 528 at 125 of
 // 128; over 8 experts Q4_K / Q6_K 34 / 39 at 128 pairs in all, 65 / 47 at 512, IQ3_S 99 / 114 at 2,048.
+// Where both types are one and a matrix has more than 1 M weights the line is higher (fixed-shape / rows
+// time, uniform and Zipf routing, 2048 / 1024, 256 experts): IQ3_S 1.01 / 0.86 at 20 pairs per
+// expert, 1.04 / 0.89 at 32, 1.11 / 0.93 at 40; Q4_K 0.99 / 1.00 at 10 (64 experts 0.96 / 0.93), 1.05 / 1.02 at
+// 13.  Smaller matrices gain from the lower one: 512 / 256, 64 experts, Q4_K 1.19 / 1.57 at 10, IQ3_S 1.12 / 1.34 at
+// 20; so do mixed types: Q6_K / Q4_K 1.06 / 1.12 at 10, Q4_K / IQ3_S 1.09 / 0.96 at 20.
 static bool prefill_takes_rows(const sabah_moe_layer_desc* L, size_t pairs) {
-    const bool iq3s = L->qt_gate == QT_IQ3_S || L->qt_down == QT_IQ3_S;
-    return pairs >= (iq3s ? 20 : 10) * (size_t)L->n_experts && pairs >= (iq3s ? 4096u : 512u);
+    const bool g3 = L->qt_gate == QT_IQ3_S, d3 = L->qt_down == QT_IQ3_S, q4 = L->qt_gate == QT_Q4_K && L->qt_down == QT_Q4_K;
+    const bool large = (size_t)L->d_model * L->d_ff > (size_t)1 << 20;
+    const int per_expert = g3 || d3 ? (large && g3 && d3 ? 32 : 20) : large && q4 ? 13 : 10;
+    return pairs >= (size_t)per_expert * L->n_experts && pairs >= (g3 || d3 ? 4096u : 512u);
 }
 
 SABAH_API int sabah_moe_prefill_layer(const sabah_moe_layer_desc* layer, const float* d_x, const int32_t* d_ids,

@@ -155,6 +155,24 @@ def test_calls_on_two_streams_and_under_capture(hip_rt, grouping):
     assert hip_rt.snapshot()["grouped_calls"] == before + 20
 
 
+# Over 8 experts a launch of few pairs is k / 256 dependent steps whatever their
+# number: the token-major kernels keep the calls below the line, by shape
+@pytest.mark.parametrize("qt,k,rows,tokens,grouped", [
+    (IQ4_XS, 2560, 640, 27, False), (IQ4_XS, 2560, 640, 60, True), (Q8_0, 2048, 768, 28, False),
+    (Q8_0, 2048, 768, 50, True), (IQ3_XXS, 4096, 1536, 16, False), (IQ3_XXS, 4096, 1536, 40, True),
+    (IQ4_XS, 4096, 1536, 9, False), (Q6_K, 2560, 640, 27, False)])
+def test_few_pairs_over_few_experts_stay_token_major(hip_rt, grouping, qt, k, rows, tokens, grouped):
+    E, K = 8, 2
+    rng = np.random.default_rng(qt + k)
+    bank = T(bank_bytes(rng, qt, E, rows, k))
+    ids = T(rng.integers(0, E, (tokens, K)).astype(np.int32))
+    x = T(rng.standard_normal((tokens, 1, k)).astype(np.float32))
+    grouping(AUTO)
+    got = mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped=grouped)
+    grouping(NEVER)
+    assert_bits_equal(got, mmid(hip_rt, bank, qt, rows, k, E, x, ids, grouped=False), "qt=%d" % qt)
+
+
 def hip_runtime():
     """The HIP runtime this process runs on."""
     with open("/proc/self/maps") as f:
