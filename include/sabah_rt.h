@@ -169,11 +169,9 @@ void sabah_slab_destroy(void);
 
 /* n elements of type qt (a whole number of blocks) at host address src,
  * decoded into n floats at host address dst.  Replaces sabah_rt_host_dequant
- * (sabah_rt.cu:3845-3847), whose decoders run on the host; here the bytes are
- * decoded on the device by the same decoders as sabah_dequant.  Synchronous;
- * callable before sabah_rt_init, like the reference's (the library is then
- * initialised on the current HIP device).  Returns -1 for an unsupported type
- * or a partial block. */
+ * (sabah_rt.cu:3845-3847); like the reference's it runs on the host, needs no GPU
+ * and no sabah_rt_init, and gives sabah_dequant's bits.  Returns -1 for an
+ * unsupported type or a partial block. */
 int sabah_rt_host_dequant(const void *src, float *dst, int qt, int n);
 
 /* Bytes of one row of n elements of type qt (0 if unsupported or n is not a

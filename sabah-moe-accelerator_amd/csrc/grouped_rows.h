@@ -14,10 +14,11 @@
 // kernels', bit for bit, in every format.
 //
 // What bounds it: decoding.  A 512-token IQ3_XXS / IQ4_NL layer (top-10 of 512,
-// 2560 / 640; 1.1 GB of weights): gate/up 285 us (2.25 TB/s; VALU busy 67 %, LDS 62 %, most of
-// it codebook look-ups), down 253 us (1.87 TB/s; VALU 63 %, LDS 30 %), two to three waves per
-// SIMD; the layer 516 us against 4,680 token-major.  A Q4_K / Q6_K layer at 1,999 tokens,
-// top-8 of 128 (125 pairs per expert): 432 us against 777 with the fixed-shape kernels.
+// 2560 / 640; 1.1 GB of weights), medians of 150 traced calls: gate/up 257 us (2.50 TB/s; VALU busy
+// 67 %, LDS 62 %, most of it codebook look-ups), down 229 us (2.06 TB/s; VALU 63 %, LDS 30 %), two to
+// three waves per SIMD, and 30 us of grouping, quantisation and combine; the layer 515 us against
+// 4,680 token-major.  A Q4_K / Q6_K layer at 1,999 tokens, top-8 of 128 (125 pairs per
+// expert): 437 us against 777 with the fixed-shape kernels.
 #pragma once
 #include "prefill_kernels.h"
 

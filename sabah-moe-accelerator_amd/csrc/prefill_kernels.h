@@ -90,7 +90,8 @@ __device__ inline int block_exclusive_scan(int v, int* tmp, int& total) {
 
 // ids a thread keeps in registers between the histogram and the scatter
 // (n_tokens * k up to 8 x 1024, or 16 x 1024 in the form for larger batches: 14 against
-// 21 us at 15,992 pairs, but 0.4 us more at 5,120); larger ones still re-read them
+// 21 us at 15,992 pairs, but 7.6 against 7.3 us at 5,120 and 5.0 against 4.2 at 602); larger
+// ones still re-read them
 constexpr int kGroupIdRegs = 8;
 
 // one workgroup of kGroupThreads; dynamic LDS: 2 * n_experts + kGroupThreads ints

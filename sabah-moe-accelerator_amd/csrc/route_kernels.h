@@ -158,8 +158,9 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
 // A pick is a wave argmax with no barrier and no LDS (the workgroup form waits for
 // both at every pick, a chain of n_used); the picks stay in lanes 0 .. n_used - 1, which
 // write them together.  Same steps and values as
-// k_route, which more experts take.  Measured at 512 experts, top-10 (us a pass of back-to-back calls):
-// 512 tokens 7.2 against 8.6, 8 tokens 7.3 against 7.7, both now the host's call.
+// k_route, which more experts take.  Measured (us a call, 100 in a replayed graph, against the workgroup
+// form): 512 experts, top-10, 512 tokens 7.1 / 8.6, one token 6.1 / 7.4; 128 experts, top-8, 512 tokens 4.5 / 6.6,
+// one token 4.0 / 5.6.  What is left is the chain of n_used picks.
 template <int PER>
 __global__ __launch_bounds__(64) void k_route_wave(RouteArgs a) {
     const int t = blockIdx.x, v = (int)threadIdx.x;
